@@ -60,7 +60,10 @@ struct GmmWs {
 // counter) sums the partials in piece order and runs the epilogue.  No workgroup waits on
 // another, and the sum does not depend on arrival order.  The dispatch assumption only
 // affects speed: any placement gives the same result.  At most kSplitItems pieces per XCD.
-constexpr int kSplitXcd = 8, kSplitItems = 32, kSplitMaxRem = 16, kSplitMaxS = 4;
+// A piece holds at least kSplitMinStages 32-k stages: exchanging the partials costs 8-15 us, so a
+// shorter reduction loses (8192 rows in 8 groups x Kred x 2048, split / whole: Kred 1408 84 / 68 us,
+// 2048 100 / 92, 4096 159 / 165, 14336 489 / 527; 2000 rows x 7168 x 1024: 80 / 175).
+constexpr int kSplitXcd = 8, kSplitItems = 32, kSplitMaxRem = 16, kSplitMaxS = 4, kSplitMinStages = 40;
 constexpr int64_t kSplitSlotFloats = 256 * 256;
 static inline int64_t gmm_ws_tiles_off(int64_t E) { return round_up((int64_t)(48 + 2 * E + 1) * 4, 256); }
 static inline int64_t gmm_max_tiles(int64_t M, int64_t E, int64_t BM) { return ceil_div(M, BM) + E + 1; }
@@ -904,6 +907,88 @@ __device__ __forceinline__ float swiglu_fast(float g, float u) {
 }
 
 
+// ---- partial tiles of the split tail ------------------------------------------------------------
+// A piece's f32 tile goes to the workspace and is read by the piece that arrives last, on any XCD.
+// Writes and reads are agent-scope accesses, which by themselves go to the level that the XCDs
+// share, so a piece only waits for its own writes before it bumps the tile's counter.  Plain stores
+// behind an agent-scope release fence write back the XCD's whole L2 in every piece, which cost
+// about 60 us a launch (2048 rows in 32 groups x 2048 x 1024: 114 us split, 49 us whole).  The
+// reads go through the idle ring (direct-to-LDS, two batches in flight): the accumulators leave few
+// registers, and reads into those few took 90 us for the 256 values a lane of gmm_w4_kernel holds.
+// Layout of a piece: wave w's rows of 64 lanes x 2 values, TM*TN*8 of them, one after the other.
+template <int TM, int TN>
+__device__ __forceinline__ void split_put(const f32x16 (&acc)[TM][TN], float* piece, int wave, int lane) {
+  float* p = piece + (wave * (TM * TN * 8)) * 128 + lane * 2;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int g = 0; g < 8; ++g)
+        __hip_atomic_store((uint64_t*)(p + ((i * TN + j) * 8 + g) * 128),
+                           (uint64_t)__float_as_uint(acc[i][j][2 * g]) |
+                               ((uint64_t)__float_as_uint(acc[i][j][2 * g + 1]) << 32),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Called by every thread of the workgroup after its split_put; true in every thread of the piece
+// that arrives last.  s_last: an int in LDS, which may be overwritten after the call.
+__device__ __forceinline__ bool split_arrive(int* counter, int npieces, int* s_last) {
+  // this wave's writes have reached the shared level (stores count in vmcnt); the barrier then
+  // covers the workgroup's, and only after it does one thread bump the counter
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(MTX_VMCNT(0));
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *s_last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == npieces - 1;
+  __syncthreads();
+  const bool last = *s_last != 0;
+  __syncthreads();
+  asm volatile("" ::: "memory");
+  return last;
+}
+// acc = the sum of the pieces in piece order, the same whatever the order of arrival.  H loads of 1 KB
+// (two rows) per wave and batch; lds: 2 * H KB per wave, idle, read by no other wave.
+template <int TM, int TN, int H>
+__device__ __forceinline__ void split_sum(f32x16 (&acc)[TM][TN], const float* pieces, int npieces, int wave, int lane,
+                                          char* lds) {
+  constexpr int LOADS = TM * TN * 4, NB = LOADS / H;  // per piece and wave; batches
+  static_assert(LOADS % H == 0, "whole batches");
+  const char* src = (const char*)(pieces + (wave * (TM * TN * 8)) * 128);
+  char* mine = lds + wave * (2 * H * 1024);
+  const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr(mine));
+  auto issue = [&](int s, int b) {
+    const uint32_t half = base + (uint32_t)(((s * NB + b) & 1) * H) * 1024u;
+    const char* from = src + (int64_t)s * (kSplitSlotFloats * 4) + b * (H * 1024) + lane * 16;
+#pragma unroll
+    for (int c = 0; c < H; ++c) gload_lds16_agent(from + c * 1024, half + c * 1024u);
+  };
+  issue(0, 0);
+  for (int s = 0; s < npieces; ++s) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const bool more = b + 1 < NB || s + 1 < npieces;
+      __builtin_amdgcn_s_waitcnt(MTX_LGKMCNT0);  // the other half's reads are done: it may be refilled
+      if (more) {
+        issue(b + 1 < NB ? s : s + 1, b + 1 < NB ? b + 1 : 0);
+        __builtin_amdgcn_s_waitcnt(MTX_VMCNT(H));
+      } else {
+        __builtin_amdgcn_s_waitcnt(MTX_VMCNT(0));
+      }
+      asm volatile("" ::: "memory");
+      const char* half = mine + (((s * NB + b) & 1) * H) * 1024 + lane * 8;
+#pragma unroll
+      for (int c = 0; c < 2 * H; ++c) {
+        const int row = b * 2 * H + c, blk = row / 8, g = row % 8;
+        const float2 v = *(const float2*)(half + c * 512);
+        f32x16& a = acc[blk / TN][blk % TN];
+        a[2 * g] = (s == 0) ? v.x : a[2 * g] + v.x;
+        a[2 * g + 1] = (s == 0) ? v.y : a[2 * g + 1] + v.y;
+      }
+      asm volatile("" ::: "memory");
+    }
+  }
+}
+
 // ---- v3: direct-to-LDS loads, 4-stage ring, transpose reads (FWD / SWIGLU / DLHS) ----------------
 // 256x256 output tile, 8 waves (2 per SIMD) with 128x64 wave tiles, BK = 32.  Every global
 // load is a global_load_lds_dwordx4 straight into a 4-deep LDS ring (no staging registers, no
@@ -1009,7 +1094,7 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       const int tx = max(0, min(per, total - xcd * per));
       const int rem = tx % p.ncu_x;
       int S = (rem > 0 && rem <= kSplitMaxRem && 2 * rem <= p.ncu_x) ? min(kSplitMaxS, p.ncu_x / rem) : 1;
-      S = min(S, max(p.Kred / BKS, 1));
+      S = min(S, max(p.Kred / BKS / kSplitMinStages, 1));
       const int nwhole = (S > 1) ? tx - rem : tx;
       if (q >= nwhole + (S > 1 ? rem * S : 0)) return;
       if (q < nwhole) {
@@ -1282,46 +1367,16 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
   __builtin_amdgcn_s_waitcnt(MTX_VMCNT(0));  // no ring load may land after the workgroup ends
 
   if (npieces > 1) {
-    // Split tail piece: publish the fp32 partial tile; the piece that arrives last (by the
-    // tile's counter) reloads every piece and adds them in piece order -- the same sum
-    // whatever the arrival order -- then runs the epilogue.  Nothing waits on another
-    // workgroup.  A lane's partial is float4 chunks, one coalesced 1 KB row per wave store.
+    // Split tail piece: publish the f32 partial tile; the piece that arrives last (by the tile's
+    // counter) adds every piece in piece order -- the same sum whatever the arrival order -- and
+    // runs the epilogue.  Nothing waits on another workgroup.
     static_assert(BM * BN <= kSplitSlotFloats, "split slot");
-    typedef __attribute__((ext_vector_type(4))) float f32x4;
-    constexpr int64_t SLOT4 = kSplitSlotFloats / 4;
     const int xcd_e = (int)(blockIdx.x & 7);
-    f32x4* part = (f32x4*)(p.split_part + (int64_t)(xcd_e * kSplitItems + split_u * npieces) * kSplitSlotFloats);
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          part[piece * SLOT4 + ((i * TN + j) * 4 + g) * NT + tid] =
-              f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __syncthreads();
-    if (tid == 0)
-      s_last = __hip_atomic_fetch_add(p.split_cnt + xcd_e * kSplitMaxRem + split_u, 1, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT) == npieces - 1;
-    __syncthreads();
-    if (!s_last) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-#pragma unroll
-    for (int s2 = 0; s2 < kSplitMaxS; ++s2) {  // unrolled: each piece's loads issue together
-      if (s2 >= npieces) break;
-      const f32x4* src = part + s2 * SLOT4;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const f32x4 v = src[((i * TN + j) * 4 + g) * NT + tid];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[i][j][4 * g + c] = (s2 == 0) ? v[c] : acc[i][j][4 * g + c] + v[c];
-          }
-    }
+    float* part = p.split_part + (int64_t)(xcd_e * kSplitItems + split_u * npieces) * kSplitSlotFloats;
+    split_put<TM, TN>(acc, part + piece * kSplitSlotFloats, wave, lane);
+    if (!split_arrive(p.split_cnt + xcd_e * kSplitMaxRem + split_u, npieces, &s_last)) return;
+    static_assert(NT / 64 * 2 * 8 * 1024 <= NSTAGE * STAGE || BM != 256, "split_sum's staging fits the ring");
+    split_sum<TM, TN, 8>(acc, part, npieces, wave, lane, lds);
   }
 
   // ---- epilogue: the MFMAs computed C^T blocks (operands swapped), so acc[i][j][4g+q] of lane
@@ -2127,42 +2182,14 @@ __device__ __forceinline__ void tile(const Args& p, char* lds, int* s_last, cons
 
   if (t.npieces > 1) {
     // split tail piece: as in gmm_v3_kernel (partials in piece order, summed by the last arrival)
-    typedef __attribute__((ext_vector_type(4))) float f32x4;
-    constexpr int64_t SLOT4 = kSplitSlotFloats / 4;
-    static_assert(TM * TN * 4 * NT <= SLOT4, "split slot");
+    static_assert(TM * TN * 16 * NT <= kSplitSlotFloats, "split slot");
     const int xcd_e = t.queue;
-    f32x4* part = (f32x4*)(p.split_part + (int64_t)(xcd_e * kSplitItems + t.split_u * t.npieces) * kSplitSlotFloats);
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          part[t.piece * SLOT4 + ((i * TN + j) * 4 + g) * NT + tid] =
-              f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __syncthreads();
-    if (tid == 0)
-      *s_last = __hip_atomic_fetch_add(p.split_cnt + xcd_e * kSplitMaxRem + t.split_u, 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT) == t.npieces - 1;
-    __syncthreads();
-    if (!*s_last) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-#pragma unroll
-    for (int s2 = 0; s2 < kSplitMaxS; ++s2) {
-      if (s2 >= t.npieces) break;
-      const f32x4* src = part + s2 * SLOT4;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const f32x4 v = src[((i * TN + j) * 4 + g) * NT + tid];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[i][j][4 * g + c] = (s2 == 0) ? v[c] : acc[i][j][4 * g + c] + v[c];
-          }
-    }
+    float* part = p.split_part + (int64_t)(xcd_e * kSplitItems + t.split_u * t.npieces) * kSplitSlotFloats;
+    split_put<TM, TN>(acc, part + t.piece * kSplitSlotFloats, wave, lane);
+    if (!split_arrive(p.split_cnt + xcd_e * kSplitMaxRem + t.split_u, t.npieces, s_last)) return;
+    constexpr int H = TM * TN * 4 < 16 ? TM * TN * 4 : (TM * TN * 4) % 16 ? 8 : 16;
+    static_assert(NT / 64 * 2 * H * 1024 <= NSTAGE * STAGE, "split_sum's staging fits the ring");
+    split_sum<TM, TN, H>(acc, part, t.npieces, wave, lane, lds);
   }
 
   // ---- epilogue: acc[i][j][4g+q] of lane l is C[row i*32 + l%32][col cbase(j) + 8g + 4(l/32) + q];
@@ -2252,7 +2279,7 @@ __global__ __launch_bounds__(256, 1) void gmm_w4_kernel(Args p) {
     if (EPI == EPI_STORE && p.split_on) {
       const int rem = tx % p.ncu_x;
       int S_ = (rem > 0 && rem <= kSplitMaxRem && 2 * rem <= p.ncu_x) ? min(kSplitMaxS, p.ncu_x / rem) : 1;
-      S_ = min(S_, max(p.Kred / v3::BKS, 1));
+      S_ = min(S_, max(p.Kred / v3::BKS / kSplitMinStages, 1));
       if (S_ > 1) {
         nwhole = tx - rem;
         S = S_;

@@ -15,6 +15,12 @@ __device__ __forceinline__ void gload_lds16(const void* gptr, uint32_t lds_base)
                : "memory", "m0");
 }
 
+// gload_lds16 at agent scope: reads what another XCD has written at agent scope.
+__device__ __forceinline__ void gload_lds16_agent(const void* gptr, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off sc1" ::"v"(gptr), "s"(lds_base)
+               : "memory", "m0");
+}
+
 // 4-byte direct global->LDS load: lane l writes LDS byte lds_base + 4*l.
 __device__ __forceinline__ void gload_lds4(const void* gptr, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gptr), "s"(lds_base)
