@@ -1027,7 +1027,14 @@ typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 #ifndef MTX_V3_SGB
 #define MTX_V3_SGB 1
 #endif
-template <int MODE, int EPI, int WM, int WN, int BM_, int NST_>
+// EDGE: widths that are multiples of 8 only (a 16-byte chunk), where a tile may hang over the
+// output's last column, the reduction may end inside a stage, or (TGMM) a tile over dW's last row.
+// Every load stays in its row's chunks: columns, reduction chunks and rows past the end re-read
+// the last valid one.  A reduction tail is masked in both operands' fragments (zeros times zeros,
+// whatever the re-read values are), columns past the end are computed and not stored.  These shapes
+// ran on the scalar-FMA kernel at about 21 TFLOP/s; the loop below without its pinned interleave,
+// plus one min per load address, keeps the MFMA tile's rate.
+template <int MODE, int EPI, int WM, int WN, int BM_, int NST_, bool EDGE = false>
 __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p) {
   using v3::BKS;
   using v3::a_off;
@@ -1055,12 +1062,13 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
   int e, r0, r1, col0, n_tile, row0 = 0;
   int piece = 0, npieces = 1, split_u = 0;  // k-piece of a split tail tile (1 piece: whole tile)
   if constexpr (MODE == TGMM) {
-    const int ntiles = p.N / BN, per_e = (p.Kd / BM) * ntiles;
+    const int ntiles = EDGE ? (p.N + BN - 1) / BN : p.N / BN;
+    const int per_e = (EDGE ? (p.Kd + BM - 1) / BM : p.Kd / BM) * ntiles;
     const int lid = blockIdx.x;
     if (lid >= p.E * per_e) return;
     e = p.order[lid / per_e];
     const int rem = lid % per_e;
-    if (p.xa > 0) {  // consecutive workgroups land on consecutive XCDs: x = rem % 8 (per_e % 8 == 0)
+    if (!EDGE && p.xa > 0) {  // consecutive workgroups land on consecutive XCDs: x = rem % 8 (per_e % 8 == 0)
       const int x = rem & 7, qq = rem >> 3, rh = (p.Kd / BM) / p.xa, rw = ntiles / p.xb;
       row0 = ((x % p.xa) * rh + qq / rw) * BM;
       n_tile = (x / p.xa) * rw + qq % rw;
@@ -1075,12 +1083,14 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       uint16_t* out = p.C + (int64_t)e * p.Kd * p.N;
       for (int i = tid; i < BM * BN / 8; i += NT) {
         const int r = i / (BN / 8), c = (i % (BN / 8)) * 8;
+        if (EDGE && (row0 + r >= p.Kd || col0 + c >= p.N)) continue;
         *(u32x4*)(out + (int64_t)(row0 + r) * p.N + col0 + c) = u32x4{0u, 0u, 0u, 0u};
       }
       return;
     }
   } else {
-    const int nn = (EPI == EPI_SWIGLU) ? (p.I / (BN / 2)) : (p.N / BN);
+    const int up = EDGE ? 1 : 0;  // a last, partial n-tile
+    const int nn = (EPI == EPI_SWIGLU) ? ((p.I + up * (BN / 2 - 1)) / (BN / 2)) : ((p.N + up * (BN - 1)) / BN);
     const int cnt = p.count[0];
     const int total = cnt * nn;
     const int pid = blockIdx.x;
@@ -1128,17 +1138,20 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       const int c0 = (EPI == EPI_SWIGLU) ? n_tile * (BN / 2) : col0;
       for (int i = tid; i < BM * ncols; i += NT) {
         const int r = r0 + i / ncols;
-        if (r < r1) p.C[(int64_t)r * p.ldc + c0 + i % ncols] = 0;
+        if (r < r1 && (!EDGE || c0 + i % ncols < p.ldc)) p.C[(int64_t)r * p.ldc + c0 + i % ncols] = 0;
       }
       return;
     }
   }
 
   // k-stages [kb0, kb0 + nk) of this workgroup (piece of npieces; the whole range when 1)
-  const int nk_all = (MODE == TGMM) ? (r1 - r0 + BKS - 1) / BKS : p.Kred / BKS;
+  const int nk_all = (MODE == TGMM) ? (r1 - r0 + BKS - 1) / BKS : (p.Kred + (EDGE ? BKS - 1 : 0)) / BKS;
   const int kb0 = piece * nk_all / npieces;
   const int nk = (piece + 1) * nk_all / npieces - kb0;
-  const int tail = (MODE == TGMM) ? (r1 - r0) - (nk - 1) * BKS : BKS;  // rows in the last step
+  // reduction elements in the last stage (BKS: no tail, or not this piece's)
+  const int tail = (MODE == TGMM) ? (r1 - r0) - (nk - 1) * BKS
+                   : (EDGE && kb0 + nk == nk_all) ? p.Kred - (nk_all - 1) * BKS : BKS;
+  constexpr bool MASKED = (MODE == TGMM) || EDGE;  // the reduction may end inside a stage
 
   // ---- per-lane global sources of the load instructions (byte offsets at k-step 0) -----
   // A row-major operand (FWD/DLHS): lane l of segment s fills row 16s + l/4, chunk slot l%4.
@@ -1149,6 +1162,7 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
   const char* Bb = (MODE == TGMM) ? (const char*)p.B : (const char*)(p.B + (int64_t)e * p.Kred * p.N);
   uint32_t aoff[A_INSTR], boff[B_INSTR];
   int arow[A_T ? A_INSTR : 1], brow[(MODE == TGMM) ? B_INSTR : 1];
+  int ak[EDGE ? A_INSTR : 1], bk[EDGE ? B_INSTR : 1];  // stage-local reduction element of the lane's chunk
 #pragma unroll
   for (int i = 0; i < A_INSTR; ++i) {
     const int seg = wave * A_INSTR + i;  // 1 KB segment of the A region
@@ -1156,7 +1170,7 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       const int k = seg * 2 + (lane >> 5), pc = lane & 31;
       const int c = pc ^ ((k & 3) << 2);
       arow[i] = r0 + k;
-      aoff[i] = (uint32_t)(row0 + c * 8) * 2u;
+      aoff[i] = (uint32_t)(EDGE ? min(row0 + c * 8, p.Kd - 8) : row0 + c * 8) * 2u;
     } else {
       const int r = seg * 16 + (lane >> 2), pc = lane & 3;
       const int c = pc ^ ((r >> 2) & 3);
@@ -1164,7 +1178,8 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       int gr = r0 + r;
       gr = gr < r1 ? gr : r1 - 1;
       if (MODE == FWD && p.gather) gr = min(max(p.gather[gr], 0) / p.gather_div, p.gather_rows - 1);
-      aoff[i] = ((uint32_t)gr * (uint32_t)p.Kred + (uint32_t)(c * 8)) * 2u;
+      aoff[i] = ((uint32_t)gr * (uint32_t)p.Kred + (EDGE ? 0u : (uint32_t)(c * 8))) * 2u;
+      if constexpr (EDGE) ak[i] = c * 8;
     }
   }
 #pragma unroll
@@ -1178,20 +1193,24 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       if (EPI == EPI_SWIGLU) {
         const int w_ = tc / WTN, within = tc % WTN;
         const int half = within / (WTN / 2), o = within % (WTN / 2);
-        gc = half * p.I + n_tile * (BN / 2) + w_ * (WTN / 2) + o;
+        const int nc = n_tile * (BN / 2) + w_ * (WTN / 2) + o;
+        gc = half * p.I + (EDGE ? min(nc, p.I - 8) : nc);
       } else {
-        gc = col0 + tc;
+        gc = EDGE ? min(col0 + tc, p.N - 8) : col0 + tc;
       }
       if constexpr (MODE == TGMM) {
         brow[i] = r0 + k;
         boff[i] = (uint32_t)gc * 2u;
       } else {
-        boff[i] = ((uint32_t)k * (uint32_t)p.N + (uint32_t)gc) * 2u;
+        boff[i] = ((EDGE ? 0u : (uint32_t)k * (uint32_t)p.N) + (uint32_t)gc) * 2u;
+        if constexpr (EDGE) bk[i] = k;
       }
     } else {
       const int r = seg * 16 + (lane >> 2), pc = lane & 3;
       const int c = pc ^ ((r >> 2) & 3);
-      boff[i] = ((uint32_t)(col0 + r) * (uint32_t)p.Kred + (uint32_t)(c * 8)) * 2u;
+      const int nr = EDGE ? min(col0 + r, p.N - 1) : col0 + r;
+      boff[i] = ((uint32_t)nr * (uint32_t)p.Kred + (EDGE ? 0u : (uint32_t)(c * 8))) * 2u;
+      if constexpr (EDGE) bk[i] = c * 8;
     }
   }
   const uint32_t a_step = BKS * 2;
@@ -1214,6 +1233,17 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       for (int i = 0; i < B_INSTR; ++i) {
         const uint32_t row = (uint32_t)min(brow[i] + kt * BKS, mlast);
         gload_lds16(Bb + row * (uint32_t)(p.N * 2) + boff[i], st + (uint32_t)A_BYTES + (wave_u * B_INSTR + i) * 1024u);
+      }
+    } else if constexpr (EDGE) {
+#pragma unroll
+      for (int i = 0; i < A_INSTR; ++i)
+        gload_lds16(Ab + aoff[i] + (uint32_t)min(kt * BKS + ak[i], p.Kred - 8) * 2u,
+                    st + (wave_u * A_INSTR + i) * 1024u);
+#pragma unroll
+      for (int i = 0; i < B_INSTR; ++i) {
+        const uint32_t off = B_T ? (uint32_t)min(kt * BKS + bk[i], p.Kred - 1) * (uint32_t)(p.N * 2)
+                                 : (uint32_t)min(kt * BKS + bk[i], p.Kred - 8) * 2u;
+        gload_lds16(Bb + boff[i] + off, st + (uint32_t)A_BYTES + (wave_u * B_INSTR + i) * 1024u);
       }
     } else {
 #pragma unroll
@@ -1264,8 +1294,8 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       }
     }
   };
-  // TGMM reduction tail: keep only the first `rem` rows of the last step (both operands, so
-  // rows of other groups never reach the accumulators).
+  // Reduction tail: keep only the first `rem` reduction elements of the last stage (both operands,
+  // so that TGMM rows of other groups and re-read chunks never reach the accumulators).
   auto mask_frags = [&](int buf, int kk, int rem) {
     const int nv = min(max(rem - kk * 16 - 8 * fhalf, 0), 8);
     u32x4 m;
@@ -1302,7 +1332,7 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
     for (int kt = 0; kt < nk; ++kt) {
       issue_stage(kt + PD);
 #if MTX_V3_SGB
-      if constexpr (FULL && MODE != TGMM) {
+      if constexpr (FULL && !MASKED) {
         // explicit interleave: one fragment read of the next substep after each MFMA
         __builtin_amdgcn_sched_barrier(0);
         read_frags(kt, 1, 1, nb);
@@ -1334,7 +1364,7 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
 #endif
       // substep 0: prefetch substep 1 of this stage
       read_frags(kt, 1, 1, nb);
-      if (MODE == TGMM && tail < BKS && kt == nk - 1) mask_frags(0, 0, tail);
+      if (MASKED && tail < BKS && kt == nk - 1) mask_frags(0, 0, tail);
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         if (!FULL && i >= nb) continue;
@@ -1345,7 +1375,7 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       // the last step this reads an unused ring slot: in bounds, and branch-free so that the
       // MFMAs below only wait for the fragments they use.
       read_frags(kt + 1, 0, 0, nb);
-      if (MODE == TGMM && tail < BKS && kt == nk - 1) mask_frags(1, 1, tail);
+      if (MASKED && tail < BKS && kt == nk - 1) mask_frags(1, 1, tail);
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         if (!FULL && i >= nb) continue;
@@ -1430,19 +1460,22 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
     obase = p.C + (int64_t)e * p.Kd * p.N + col0;
     ld = p.N;
     rbase = row0;
-    rlimit = row0 + BM;
+    rlimit = EDGE ? min(row0 + BM, p.Kd) : row0 + BM;
   } else {
     obase = p.C + ((EPI == EPI_SWIGLU) ? n_tile * (BN / 2) : col0);
     ld = p.ldc;
     rbase = r0;
     rlimit = r1;
   }
+  // first output column of the tile, and the columns of it that exist
+  const int ocol0 = (MODE != TGMM && EPI == EPI_SWIGLU) ? n_tile * (BN / 2) : col0;
+  const int ocols = (MODE == TGMM ? p.N : p.ldc) - ocol0;
   constexpr int RPI = 64 / OCH;  // rows per wave instruction
   for (int rr = wave * RPI + lane / OCH; rr < BM; rr += NT / OCH) {
     const int c = lane % OCH;
     const u32x4 v = *(const u32x4*)(lds + rr * OROW + ((c ^ (rr & 15)) << 4));
     const int row = rbase + rr;
-    if (row < rlimit) *(u32x4*)(obase + (int64_t)row * ld + c * 8) = v;
+    if (row < rlimit && (!EDGE || c * 8 < ocols)) *(u32x4*)(obase + (int64_t)row * ld + c * 8) = v;
   }
 }
 
@@ -2431,6 +2464,14 @@ static int launch_v3(const mf::Args& a, int64_t grid, hipStream_t st) {
 #ifndef MTX_V3S_NST
 #define MTX_V3S_NST 3
 #endif
+// The 256-row tiles at widths that are multiples of 8 only (gmm_v3_kernel's EDGE form).
+template <int MODE, int EPI>
+static int launch_v3_edge(const mf::Args& a, int64_t grid, hipStream_t st) {
+  if (grid <= 0) return MTX_OK;
+  grid = round_up(grid, 8);
+  hipLaunchKernelGGL((mf::gmm_v3_kernel<MODE, EPI, 2, 4, 256, 4, true>), dim3((unsigned)grid), dim3(512), 0, st, a);
+  return check_launch();
+}
 // Persistent plain-store kernel for reductions of 4 .. MTX_V4P_MAX_STAGES 32-k stages (0: never):
 // one workgroup per CU, each walking its XCD's share of the tile list.  Measured against
 // gmm_v3_kernel on the same box (E = 8, M = 16384, N = 4096): +36 % at Kred 512, +10 % at 1024,
@@ -2546,15 +2587,10 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
   // bf16 MFMA eligibility
   const bool aligned = ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
   if (gath && !(dtype == MTX_BF16 && aligned && Kred % mf::BK == 0 && Kred > 0)) return MTX_ERR_UNSUPPORTED;
-  if (dtype == MTX_BF16 && aligned && Kred % mf::BK == 0 && Kred > 0) {
+  auto base_args = [&]() {
     mf::Args a;
     a.A = (const uint16_t*)x;
     a.B = (const uint16_t*)w;
-    if (gath) {
-      a.gather = gather;
-      a.gather_div = (int)gather_div;
-      a.gather_rows = (int)gather_rows;
-    }
     a.C = (uint16_t*)out;
     a.count = wsp.count;
     a.offsets = wsp.offsets;
@@ -2567,6 +2603,15 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
     a.ldc = (int)out_cols;
     a.I = (int)I;
     a.E = (int)E;
+    return a;
+  };
+  if (dtype == MTX_BF16 && aligned && Kred % mf::BK == 0 && Kred > 0) {
+    mf::Args a = base_args();
+    if (gath) {
+      a.gather = gather;
+      a.gather_div = (int)gather_div;
+      a.gather_rows = (int)gather_rows;
+    }
     // A tile group of gm m-tiles runs against a few n-tiles at a time on one XCD.  With several
     // m-tiles per expert, 8 balances the re-reads of x and W through L2; with about one m-tile
     // per expert (W is read once whatever the order) 1 keeps each x tile in L2 while all its
@@ -2645,7 +2690,9 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
       return mode == 0 ? launch_mfma<128, 256, 1, 2, mf::FWD, mf::EPI_STORE>(a, grid, st)
                        : launch_mfma<128, 256, 1, 2, mf::DLHS, mf::EPI_STORE>(a, grid, st);
     }
-    if (mode != 2 && Nout % 128 == 0) {
+    // Nout a multiple of 128 but not of 256: the ring kernel's EDGE form below is faster (8192 rows
+    // in 8 groups, 1024 x 1408: 55 -> 37 us, its dlhs 49 -> 38 us); this one keeps what that cannot take
+    if (mode != 2 && Nout % 128 == 0 && (!v3ok || (uintptr_t)out % 16 != 0)) {
       rc = launch_build_tiles(gs, E, M, 128, wsp, st);
       if (rc) return rc;
       const int64_t grid = gmm_max_tiles(M, E, 128) * (Nout / 128);
@@ -2653,8 +2700,33 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
                        : launch_mfma<128, 128, 2, 2, mf::DLHS, mf::EPI_STORE>(a, grid, st);
     }
   }
-  // generic path (exact fp32 FMA; also bf16 shapes the MFMA tiling does not cover)
   if (gath) return MTX_ERR_UNSUPPORTED;
+  // bf16 with widths that are multiples of 8: the 256-row MFMA tiles with partial n-tiles and
+  // reduction tails.  16-byte loads and stores need aligned rows (hence the 8, and out's alignment)
+  // and the kernel's operand offsets are 32-bit.  Against the FMA kernel (6124 rows in 32 skewed
+  // groups): 1536 x 2*704 with SwiGLU 1810 -> 77 us; the smallest shapes are equal.
+  if (dtype == MTX_BF16 && aligned && (uintptr_t)out % 16 == 0 && Kred > 0 && Kred % 8 == 0 && Nout % 8 == 0 &&
+      out_cols % 8 == 0 && M * Kred * 2 < (int64_t(1) << 32) && Kred * Nout * 2 < (int64_t(1) << 32)) {
+    mf::Args a = base_args();
+    a.gm = tile_group > 0 ? tile_group : ((M / E) <= 256 ? MTX_GM_SMALL : 8);
+    const int ncu = cus_per_xcd();
+    const bool split = mode != 2 && ws_bytes >= gmm_ws_split_off(M, E) + gmm_ws_split_bytes() && ncu >= 2 &&
+                       ncu <= kSplitItems;
+    if (split) {
+      a.split_on = 1;
+      a.split_cnt = wsp.split_cnt;
+      a.split_part = wsp.split_part;
+      a.ncu_x = ncu;
+    }
+    rc = launch_build_tiles(gs, E, M, 256, wsp, st, false, split, a.gm == 1 ? MTX_SPREAD_MIN : 0);
+    if (rc) return rc;
+    const int64_t nn = (mode == 2) ? ceil_div(I, 128) : ceil_div(Nout, 256);
+    const int64_t grid = round_up(gmm_max_tiles(M, E, 256) * nn, 8) + (split ? 8 * (int64_t)ncu : 0);
+    if (mode == 2) return launch_v3_edge<mf::FWD, mf::EPI_SWIGLU>(a, grid, st);
+    return mode == 0 ? launch_v3_edge<mf::FWD, mf::EPI_STORE>(a, grid, st)
+                     : launch_v3_edge<mf::DLHS, mf::EPI_STORE>(a, grid, st);
+  }
+  // generic path (exact fp32 FMA; also bf16 shapes the MFMA tiling does not cover)
   rc = launch_build_tiles(gs, E, M, kMinBM, wsp, st);
   if (rc) return rc;
   const int64_t ntile_max = gmm_max_tiles(M, E, kMinBM);
@@ -2802,7 +2874,7 @@ extern "C" int mtx_tgmm(const void* x, const void* g, const int32_t* group_sizes
   rc = launch_build_tiles(group_sizes, E, M, kMinBM, wsp, st, true);
   if (rc) return rc;
   const bool aligned = ((uintptr_t)x % 16 == 0) && ((uintptr_t)g % 16 == 0);
-  if (dtype == MTX_BF16 && aligned && K % 128 == 0 && N % 128 == 0 && M > 0) {
+  auto tgmm_args = [&]() {
     mf::Args a;
     a.A = (const uint16_t*)x;
     a.B = (const uint16_t*)g;
@@ -2819,6 +2891,10 @@ extern "C" int mtx_tgmm(const void* x, const void* g, const int32_t* group_sizes
     a.I = 0;
     a.E = (int)E;
     a.gm = 8;
+    return a;
+  };
+  if (dtype == MTX_BF16 && aligned && K % 128 == 0 && N % 128 == 0 && M > 0) {
+    mf::Args a = tgmm_args();
     if (K % 256 == 0 && N % 256 == 0 && M * K * 2 < (int64_t(1) << 32) && M * N * 2 < (int64_t(1) << 32)) {
       // XCD rectangles of each expert's tile grid: xa x xb = 8, xa | K/256, xb | N/256, fewest
       // blocks per XCD
@@ -2844,8 +2920,17 @@ extern "C" int mtx_tgmm(const void* x, const void* g, const int32_t* group_sizes
       const int64_t grid = round_up(E * (K / 256) * (N / 256), 8);
       return launch_mfma<256, 256, 2, 2, mf::TGMM, mf::EPI_STORE>(a, grid, st);
     }
-    const int64_t grid = round_up(E * (K / 128) * (N / 128), 8);
-    return launch_mfma<128, 128, 2, 2, mf::TGMM, mf::EPI_STORE>(a, grid, st);
+    // (8192 rows in 8 groups, 1408 x 1024: 58 us here, 38 us in the ring kernel's EDGE form below)
+    if ((uintptr_t)dw % 16 != 0 || M * K * 2 >= (int64_t(1) << 32) || M * N * 2 >= (int64_t(1) << 32)) {
+      const int64_t grid = round_up(E * (K / 128) * (N / 128), 8);
+      return launch_mfma<128, 128, 2, 2, mf::TGMM, mf::EPI_STORE>(a, grid, st);
+    }
+  }
+  if (dtype == MTX_BF16 && aligned && (uintptr_t)dw % 16 == 0 && K % 8 == 0 && N % 8 == 0 && M > 0 &&
+      M * K * 2 < (int64_t(1) << 32) && M * N * 2 < (int64_t(1) << 32)) {
+    // widths that are multiples of 8: partial tiles at dW's last rows and columns (6124 rows in 32
+    // skewed groups, 704 x 1536: 1994 us in the FMA kernel, 50 us here)
+    return launch_v3_edge<mf::TGMM, mf::EPI_STORE>(tgmm_args(), E * ceil_div(K, 256) * ceil_div(N, 256), st);
   }
   dim3 grid((unsigned)E, (unsigned)ceil_div(K, 64), (unsigned)ceil_div(N, 64));
   if (dtype == MTX_F32)
