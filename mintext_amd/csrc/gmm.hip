@@ -26,6 +26,7 @@
 // byte offsets.
 // f32 path (and shapes the MFMA tiling does not cover): an LDS-tiled exact-fp32 FMA kernel.
 #include "common.h"
+#include "gmm_thin.h"
 #include "lds_dma.h"
 #include <type_traits>
 #include <algorithm>
@@ -2587,6 +2588,27 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
   // bf16 MFMA eligibility
   const bool aligned = ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
   if (gath && !(dtype == MTX_BF16 && aligned && Kred % mf::BK == 0 && Kred > 0)) return MTX_ERR_UNSUPPORTED;
+  // groups of few rows (decoding): the weight-streaming kernel, with its own row lookup
+  const bool ring_gather = !gath || (Kred % mf::v3::BKS == 0 && gather_rows * Kred * 2 < (int64_t(1) << 32) &&
+                                     Kred * Nout * 2 < (int64_t(1) << 32) &&
+                                     ((mode == 2 && I % 128 == 0) || (mode == 0 && Nout % 256 == 0)));
+  if (dtype == MTX_BF16 && aligned && (uintptr_t)out % 16 == 0 && mode != 1 && ring_gather &&
+      gmm_thin_ok(M, E, Kred, Nout, I)) {
+    ThinArgs t;
+    t.A = (const uint16_t*)x;
+    t.W = (const uint16_t*)w;
+    t.C = (uint16_t*)out;
+    t.gs = gs;
+    t.gather = gather;
+    t.gather_div = (int)gather_div;
+    t.gather_rows = (int)gather_rows;
+    t.M = (int)M;
+    t.E = (int)E;
+    t.Kred = (int)Kred;
+    t.N = (int)Nout;
+    t.I = (int)(mode == 2 ? I : 0);
+    return launch_gmm_thin(t, st);
+  }
   auto base_args = [&]() {
     mf::Args a;
     a.A = (const uint16_t*)x;
