@@ -1,4 +1,5 @@
-// Grouped GEMM for groups of few rows (gmm_thin.hip); called by the dispatch in gmm.hip.
+// Grouped GEMMs for groups of few rows: bf16 (gmm_thin.hip, called by the dispatch in gmm.hip) and
+// blockwise fp8 (gmm_fp8_thin.hip, called by the one in fp8.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
@@ -20,5 +21,25 @@ struct ThinArgs {
 // in 16-byte chunks, 16-byte aligned operands (the caller checks), few rows per group on average.
 bool gmm_thin_ok(int64_t M, int64_t E, int64_t Kred, int64_t N, int64_t I);
 int launch_gmm_thin(const ThinArgs& a, hipStream_t st);
+
+struct Fp8ThinArgs {
+  const uint8_t* xq;  // [M or gather_rows][K] e4m3
+  const float* xs;    // [M or gather_rows][K/128]
+  const uint8_t* wq;  // [E][N][K] e4m3
+  const float* ws;    // [E][N/128][K/128]
+  const int32_t* gs;
+  uint16_t* out;      // plain: bf16 [M][N]; SwiGLU: bf16 [M][I] or nullptr
+  uint8_t* outq;      // SwiGLU: e4m3 [M][I]
+  float* outs;        // SwiGLU: [M][I/128]
+  const int32_t* gather;
+  int gather_div, gather_rows;
+  int M, E, K, N;
+  int I;              // SwiGLU: N = 2 I, gate rows first; 0: plain store
+};
+
+// Whether launch_fp8_thin is the kernel for M rows in E groups of K x N (K a multiple of 128).
+bool fp8_thin_ok(int64_t M, int64_t E);
+// p2: power-of-two scales (the MFMA's E8M0 operands); otherwise f32 scales.
+int launch_fp8_thin(const Fp8ThinArgs& a, bool p2, hipStream_t st);
 
 }  // namespace mtx

@@ -12,7 +12,7 @@
 // group_sizes itself: no tile list, no launch before this one.
 #include "common.h"
 #include "gmm_thin.h"
-#include <algorithm>
+#include "thin_rows.h"
 
 namespace mtx {
 namespace thin {
@@ -53,79 +53,15 @@ __global__ __launch_bounds__(NW * 64) void gmm_thin_kernel(ThinArgs p) {
   constexpr bool SWIGLU = FORM != PLAIN;
   constexpr int KW = FORM == WIDE ? NW / 2 : NW;  // waves that share a reduction
   __shared__ __attribute__((aligned(16))) float part[NW][16][PADN];
-  __shared__ int s_wave[NW];
-  __shared__ int s_tile[3];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ocols = SWIGLU ? p.I : p.N;
   constexpr int OB = FORM == NARROW ? BN / 2 : BN;  // output columns per workgroup
   const int nn = (ocols + OB - 1) / OB;
   const int mt = blockIdx.x / nn, nt = blockIdx.x % nn;
 
-  // ---- the rows of m-tile mt: groups in order, ceil(size / MT) m-tiles each, then the rows past the
-  // last group (e = -1, written as zeros).  Thread t scans the groups [t*per, (t+1)*per).
-  {
-    const int per = (p.E + NT - 1) / NT;
-    const int e0 = min(tid * per, p.E), e1 = min(e0 + per, p.E);
-    int tiles = 0, rows = 0;  // sums stay below 2^31: E <= 1024 groups, each clamped to M < 2^20 rows
-    for (int e = e0; e < e1; ++e) {
-      const int g = min(max(p.gs[e], 0), p.M);
-      tiles += (g + MT - 1) / MT;
-      rows += g;
-    }
-    int ti = tiles, ri = rows;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int a = __shfl_up(ti, off), b = __shfl_up(ri, off);
-      if (lane >= off) {
-        ti += a;
-        ri += b;
-      }
-    }
-    __shared__ int s_rows[NW];
-    if (lane == 63) {
-      s_wave[wave] = ti;
-      s_rows[wave] = ri;
-    }
-    if (tid == 0) s_tile[0] = -2;
-    __syncthreads();
-    int t0 = ti - tiles, r0 = ri - rows, tsum = 0, rsum = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const int a = s_wave[w], b = s_rows[w];
-      if (w < wave) {
-        t0 += a;
-        r0 += b;
-      }
-      tsum += a;
-      rsum += b;
-    }
-    if (mt >= t0 && mt < t0 + tiles) {
-      int t = t0, r = r0;
-      for (int e = e0; e < e1; ++e) {
-        const int g = min(max(p.gs[e], 0), p.M), n = (g + MT - 1) / MT;
-        if (mt < t + n) {
-          const int b = r + (mt - t) * MT;
-          s_tile[0] = e;
-          s_tile[1] = min(b, p.M);
-          s_tile[2] = min(min(b + MT, r + g), p.M);
-          break;
-        }
-        t += n;
-        r += g;
-      }
-    }
-    if (tid == 0 && mt >= tsum) {
-      const int b = min(rsum, p.M) + (mt - tsum) * MT;
-      if (b < p.M) {
-        s_tile[0] = -1;
-        s_tile[1] = b;
-        s_tile[2] = min(b + MT, p.M);
-      }
-    }
-    __syncthreads();
-  }
-  const int e = s_tile[0], r0 = s_tile[1], r1 = s_tile[2];
-  if (e == -2 || r0 >= r1) return;
+  const ThinRows rows = thin_rows<MT, NT>(p.gs, p.E, p.M, mt);
+  const int e = rows.e, r0 = rows.r0, r1 = rows.r1;
+  if (e == -2) return;
   if (e < 0) {
     for (int i = tid; i < MT * OB; i += NT) {
       const int r = r0 + i / OB, c = nt * OB + i % OB;
@@ -198,13 +134,21 @@ __global__ __launch_bounds__(NW * 64) void gmm_thin_kernel(ThinArgs p) {
     Chunk c0, c1;
 #pragma unroll
     for (int b = 0; b < TB; ++b) c0.x[b] = c1.x[b] = u32x4{0u, 0u, 0u, 0u};
-    // chunks past the end re-read the last one and are not used
-    load(c0, min(kw, nk - 1));
-    for (int ck = kw; ck < nk; ck += 2 * KW) {
-      load(c1, min(ck + KW, nk - 1));
+    // the loop's loads are unconditional, so that the waits count them; the last one or two chunks follow
+    if (kw < nk) load(c0, kw);
+    int ck = kw;
+    for (; ck + 2 * KW < nk; ck += 2 * KW) {
+      load(c1, ck + KW);
       use(c0, ck);
-      load(c0, min(ck + 2 * KW, nk - 1));
-      if (ck + KW < nk) use(c1, ck + KW);
+      load(c0, ck + 2 * KW);
+      use(c1, ck + KW);
+    }
+    if (ck + KW < nk) {
+      load(c1, ck + KW);
+      use(c0, ck);
+      use(c1, ck + KW);
+    } else if (ck < nk) {
+      use(c0, ck);
     }
   }
 
@@ -254,10 +198,11 @@ static int launch(const ThinArgs& a, int64_t grid, bool stream, hipStream_t st) 
 }  // namespace thin
 
 // Up to 16 rows per group on average.  128 groups, 2048 x 1536 with SwiGLU / 768 x 2048, us here and
-// in the ring kernel (weights cold): 8 rows 12.6 / 35.2 and 8.3 / 27.6, 512 rows 117 / 141 and
-// 66 / 118 (6.5 TB/s), 2048 rows (a mean of 16) 131 / 146 and 79 / 119, but 6144 rows 251 / 155: groups
-// then outgrow the m-tile of 32 rows and stream their weights again.  8 groups, 4096 x 2*14336 and
-// 14336 x 4096: 74 rows 306 / 344 and 144 / 226, 400 rows 525 / 372.
+// in the ring kernel: 8 rows 12.3 / 35.0 and 7.8 / 27.6, 512 rows 116 / 141 and 63 / 118 (6.7 and 6.2
+// TB/s), 2048 rows (a mean of 16) 129 / 147 and 79 / 119, the same with Zipf loads 154 / 158 and
+// 77 / 124, but 6144 rows 251 / 155: groups then outgrow the m-tile of 32 rows and stream their
+// weights again.  8 groups, 4096 x 2*14336 and 14336 x 4096: 74 rows 306 / 344 and 144 / 226, 400 rows
+// 525 / 372.
 constexpr int64_t kThinMaxMean = 16;
 
 bool gmm_thin_ok(int64_t M, int64_t E, int64_t Kred, int64_t N, int64_t I) {
@@ -269,7 +214,7 @@ bool gmm_thin_ok(int64_t M, int64_t E, int64_t Kred, int64_t N, int64_t I) {
 int launch_gmm_thin(const ThinArgs& a, hipStream_t st) {
   // rows per m-tile: 16 when the groups hold a row or two on average, else 32
   const int64_t MT = a.M <= 2 * (int64_t)a.E ? 16 : 32;
-  const int64_t mtiles = std::min<int64_t>(a.E, a.M) + a.M / MT + 1;  // groups with rows, full tiles, the rest
+  const int64_t mtiles = thin_max_tiles(a.M, a.E, MT);
   const int64_t bytes = mtiles * a.Kred * a.N * 2;                   // of weights, at most
   // Half the 256 MB memory-side cache or more: nothing of the weights is found there again by the
   // time they are next used, and loads that do not allocate in it run at 6.2-6.7 TB/s instead of
