@@ -12,6 +12,7 @@
 // f32 on the partial sums) and a bf16 output, or -- for the gate_up GEMM -- the SwiGLU and
 // a 1x128 re-quantisation of its output fused into the epilogue.
 #include "common.h"
+#include "gmm_thin.h"
 #include "lds_dma.h"
 #include "fp8_tile.h"
 #include <type_traits>
@@ -1221,6 +1222,28 @@ static inline int64_t f8_ws_bytes(int64_t M, int64_t E, int64_t BM) {
   return 256 + (ceil_div(M, BM) + E + 1) * (int64_t)sizeof(MTileF8);
 }
 
+// Groups of few rows (decoding): the weight-streaming kernel, with its own row lookup.
+static int launch_fp8_few(const f8::Args& a, const int32_t* gs, int64_t E, bool p2, hipStream_t st) {
+  Fp8ThinArgs t{};
+  t.xq = a.xq;
+  t.xs = a.xs;
+  t.wq = a.wq;
+  t.ws = a.ws;
+  t.gs = gs;
+  t.out = a.out;
+  t.outq = a.outq;
+  t.outs = a.outs;
+  t.gather = a.gather;
+  t.gather_div = a.gather_div;
+  t.gather_rows = a.gather_rows;
+  t.M = a.M;
+  t.E = (int)E;
+  t.K = a.K;
+  t.N = a.N;
+  t.I = a.I;
+  return launch_fp8_thin(t, p2, st);
+}
+
 // Power-of-two scales (p2): the persistent kernel with the block scales as the MFMA's E8M0
 // operands; it needs K >= 256 and 32-bit operand offsets (MTX_ERR_UNSUPPORTED otherwise).
 template <int EPI>
@@ -1228,6 +1251,7 @@ static int launch_fp8_v4_p2(const f8::Args& a, const int32_t* gs, int64_t E, int
   const int64_t a_rows = a.gather ? a.gather_rows : a.M;
   const bool off32 = a_rows * a.K < (int64_t(1) << 32) && (int64_t)a.N * a.K < (int64_t(1) << 32);
   if (!(off32 && a.K >= 256)) return MTX_ERR_UNSUPPORTED;
+  if (fp8_thin_ok(a.M, E)) return launch_fp8_few(a, gs, E, true, st);
   int* count = (int*)ws;
   MTileF8* tiles = (MTileF8*)((char*)ws + 256);
   hipLaunchKernelGGL(f8::build_tiles_f8_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, a.M, 256, count, tiles);
@@ -1248,6 +1272,7 @@ static int launch_fp8(const f8::Args& a, const int32_t* gs, int64_t E, int64_t n
   const bool off32 = a_rows * a.K < (int64_t(1) << 32) && (int64_t)a.N * a.K < (int64_t(1) << 32);
   if (a.gather && !(off32 && a.K >= 256)) return MTX_ERR_UNSUPPORTED;  // gathered rows: v4 kernel only
   if (off32 && a.K >= 256) {
+    if (fp8_thin_ok(a.M, E)) return launch_fp8_few(a, gs, E, false, st);
     int* count = (int*)ws;
     MTileF8* tiles = (MTileF8*)((char*)ws + 256);
     hipLaunchKernelGGL(f8::build_tiles_f8_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, a.M, 256, count, tiles);
