@@ -24,7 +24,7 @@
 // idle ring and writes whole 128-byte lines.  gmm_mfma_kernel, an earlier register-staged design
 // (two LDS buffers, 8x8 register transposes), runs only the shapes whose operands exceed 32-bit
 // byte offsets.
-// f32 path (and shapes the MFMA tiling does not cover): an LDS-tiled exact-fp32 FMA kernel.
+// f32 path (and bf16 widths that are no multiple of 8): f32 MFMA tiles staged through LDS.
 #include "common.h"
 #include "gmm_thin.h"
 #include "lds_dma.h"
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
   }
 }
 
-// ---- generic exact-fp32 path ------------------------------------------------------------------
+// ---- element access of the kernels that take either type --------------------------------------
 template <typename T> __device__ __forceinline__ float gld(const T* p, int64_t i);
 template <> __device__ __forceinline__ float gld<float>(const float* p, int64_t i) { return p[i]; }
 template <> __device__ __forceinline__ float gld<uint16_t>(const uint16_t* p, int64_t i) { return bf16_to_f32(p[i]); }
@@ -315,163 +315,197 @@ template <typename T> __device__ __forceinline__ void gst(T* p, int64_t i, float
 template <> __device__ __forceinline__ void gst<float>(float* p, int64_t i, float v) { p[i] = v; }
 template <> __device__ __forceinline__ void gst<uint16_t>(uint16_t* p, int64_t i, float v) { p[i] = f32_to_bf16(v); }
 
+// ---- f32 path on the f32 matrix cores -------------------------------------------------------------
+// 64x64 output tiles, 4 waves of 32x32, 32-deep reduction stages through LDS with the next stage's
+// operands loaded into registers meanwhile.  v_mfma_f32_32x32x2_f32 multiplies and accumulates in f32
+// at twice the rate of the unpacked FMAs, and needs two LDS values per lane for 64 cycles of work
+// where the FMA tile needed 8 per 64.  Measured, FMA kernel -> this: 16384 rows in 16 groups x 1024 x
+// 1024 forward 710 -> 329 us (104 TFLOP/s), dlhs 850 -> 332, tgmm 774 -> 333; 4000 rows in 16 skewed
+// groups, 512 x 768: 95 -> 45, 150 -> 50, 320 -> 54; 512 rows in 8 groups, 256 x 128: 30 -> 13.  Any
+// size and alignment: VEC = 4 moves 16 bytes at a time (every row 16-byte aligned), VEC = 1 single
+// values.  Values past the end are zeros in both operands.  T: float, or bf16 where the rows have no
+// alignment that the bf16 matrix-core kernels take (VEC = 1).
+namespace f32mm {
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+constexpr int BM = 64, BN = 64, KS = 32, NT = 256;
+constexpr int RS = KS + 4;  // LDS row of a k-contiguous operand: [64][RS]
+constexpr int CS = 64 + 8;  // LDS row of an operand stored [k][64]: the half-waves' rows 4 k apart differ by 32 banks
+constexpr int TILE = 64 * RS > KS * CS ? 64 * RS : KS * CS;
+
+// One operand tile of 64 rows x KS reduction elements (COLS = false: the reduction contiguous in
+// memory) or KS reduction elements x 64 columns (COLS = true).  at(r, c, v) says whether row r,
+// column c exists and where it is.
+template <typename T, bool COLS, int VEC>
+struct Stage {
+  static_assert(VEC == 1 || std::is_same<T, float>::value, "16-byte loads are of f32");
+  static constexpr int W = COLS ? 64 : KS, H = COLS ? KS : 64, N = W * H / NT / VEC;
+  float v[N][VEC];
+  template <typename At>
+  __device__ __forceinline__ void load(At at, int tid) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int q = tid + u * NT, r = q / (W / VEC), c = q % (W / VEC) * VEC;
+      const T* src = at(r, c);
+      if constexpr (VEC == 4) {
+        const f32x4 x = src ? *(const f32x4*)src : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[u][i] = x[i];
+      } else {
+        v[u][0] = src ? gld<T>(src, 0) : 0.0f;
+      }
+    }
+  }
+  __device__ __forceinline__ void store(float* lds, int tid) const {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int q = tid + u * NT, r = q / (W / VEC), c = q % (W / VEC) * VEC;
+      float* dst = lds + r * (COLS ? CS : RS) + c;
+      if constexpr (VEC == 4) *(f32x4*)dst = f32x4{v[u][0], v[u][1], v[u][2], v[u][3]};
+      else *dst = v[u][0];
+    }
+  }
+};
+// The 16 operand values of a lane for a stage: row or column x0 + lane % 32; MFMA m of the stage
+// multiplies reduction elements k = 8 (m / 4) + 4 (lane / 32) + m % 4 (the same for both operands).
+template <bool COLS>
+__device__ __forceinline__ void fragment(const float* lds, int x0, int lane, float f[16]) {
+  const int x = x0 + (lane & 31), h = lane >> 5;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if constexpr (COLS) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f[4 * q + i] = lds[(8 * q + 4 * h + i) * CS + x];
+    } else {
+      const f32x4 v = *(const f32x4*)(lds + x * RS + 8 * q + 4 * h);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f[4 * q + i] = v[i];
+    }
+  }
+}
+// acc of lane l, element v: row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32 of the wave's 32x32 tile.
+template <typename T, bool ACOLS, bool BCOLS, int VEC, typename AtA, typename AtB>
+__device__ __forceinline__ void mainloop(f32x16& acc, int nk, float* as, float* bs, AtA at_a, AtB at_b) {
+  const int tid = threadIdx.x, lane = tid & 63, wm = (tid >> 6) >> 1, wn = (tid >> 6) & 1;
+  Stage<T, ACOLS, VEC> a;
+  Stage<T, BCOLS, VEC> b;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+  auto load = [&](int s) {
+    a.load([&](int r, int c) { return at_a(r, c, s); }, tid);
+    b.load([&](int r, int c) { return at_b(r, c, s); }, tid);
+  };
+  if (nk > 0) load(0);
+  // one LDS buffer: a second one saves a barrier a stage but halves the workgroups per CU (5-9 % slower)
+  for (int s = 0; s < nk; ++s) {
+    a.store(as, tid);
+    b.store(bs, tid);
+    __syncthreads();
+    if (s + 1 < nk) load(s + 1);
+    float fa[16], fb[16];
+    fragment<ACOLS>(as, wm * 32, lane, fa);
+    fragment<BCOLS>(bs, wn * 32, lane, fb);
+#pragma unroll
+    for (int m = 0; m < 16; ++m) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[m], fb[m], acc, 0, 0, 0);
+    __syncthreads();
+  }
+}
+
 // MODE 0: C[r,n] = sum_k A[r,k] W[e,k,n]   (W: [E][Kred][Nout])
 // MODE 1: C[r,n] = sum_k A[r,k] W[e,n,k]   (W: [E][Nout][Kred], the dlhs transpose)
 // MODE 2: as MODE 0 with Nout = 2I, fused SwiGLU: the 64-column tile holds 32 gate columns
 //         and the 32 matching up columns; C[r,j] = silu(gate) * up, C is [M][I].
-template <typename T, int MODE>
-__global__ __launch_bounds__(256) void gmm_generic_kernel(const T* __restrict__ A, const T* __restrict__ W,
-                                                          const MTile* __restrict__ tiles,
-                                                          const int* __restrict__ count, int64_t Kred,
-                                                          int64_t Nout, T* __restrict__ C) {
-  constexpr int KS = 32;  // reduction elements per step; the next step's operands load during this one
-  __shared__ float As[KS][65];
-  __shared__ float Bs[KS][65];
+template <typename T, int MODE, int VEC>
+__global__ __launch_bounds__(NT) void gmm_kernel(const T* __restrict__ A, const T* __restrict__ W,
+                                                 const MTile* __restrict__ tiles, const int* __restrict__ count,
+                                                 int64_t Kred, int64_t Nout, T* __restrict__ C) {
+  __shared__ __attribute__((aligned(16))) float as[TILE], bs[TILE];
   if ((int)blockIdx.x >= count[0]) return;
   const MTile t = tiles[blockIdx.x];
   const int64_t I = Nout / 2;
-  const int64_t n0 = (MODE == 2) ? (int64_t)blockIdx.y * 32 : (int64_t)blockIdx.y * 64;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  constexpr int OB = MODE == 2 ? 32 : 64;  // output columns of the tile
+  const int64_t n0 = (int64_t)blockIdx.y * OB, ldc = MODE == 2 ? I : Nout;
+  const int tid = threadIdx.x, lane = tid & 63, wm = (tid >> 6) >> 1, wn = (tid >> 6) & 1;
   if (t.e < 0) {
-    const int ncol = (MODE == 2) ? 32 : 64;
-    const int64_t ldc = (MODE == 2) ? I : Nout;
-    for (int i = threadIdx.x; i < 64 * ncol; i += 256) {
-      const int64_t r = t.r0 + i / ncol, n = n0 + i % ncol;
+    for (int i = tid; i < BM * OB; i += NT) {
+      const int64_t r = t.r0 + i / OB, n = n0 + i % OB;
       if (r < t.r1 && n < ldc) gst<T>(C, r * ldc + n, 0.0f);
     }
     return;
   }
   const T* We = W + (int64_t)t.e * Kred * Nout;
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-  // per thread and step: 8 elements of the 64 x KS A tile (k fastest: coalesced rows) and 8 of
-  // the KS x 64 W tile (n fastest), zero outside the group / matrix
-  constexpr int PT = KS * 64 / 256;
-  float ra[PT], rb[PT];
-  auto load = [&](int64_t k0) {
-#pragma unroll
-    for (int u = 0; u < PT; ++u) {
-      const int i = threadIdx.x + u * 256;
-      const int kk = i % KS, rr = i / KS;
-      const int64_t r = t.r0 + rr, k = k0 + kk;
-      ra[u] = (r < t.r1 && k < Kred) ? gld<T>(A, r * Kred + k) : 0.0f;
-      const int nn = i % 64, kb = i / 64;
-      const int64_t k2 = k0 + kb;
-      float b = 0.0f;
-      if (MODE == 2) {
-        const int64_t j = n0 + (nn & 31);
-        const int64_t n = (nn < 32) ? j : I + j;
-        if (j < I && k2 < Kred) b = gld<T>(We, k2 * Nout + n);
-      } else {
-        const int64_t n = n0 + nn;
-        if (n < Nout && k2 < Kred) b = (MODE == 0) ? gld<T>(We, k2 * Nout + n) : gld<T>(We, n * Kred + k2);
-      }
-      rb[u] = b;
-    }
+  auto at_a = [&](int r, int c, int s) -> const T* {
+    const int64_t row = t.r0 + r, k = (int64_t)s * KS + c;
+    return row < t.r1 && k < Kred ? A + row * Kred + k : nullptr;
   };
-  load(0);
-  for (int64_t k0 = 0; k0 < Kred; k0 += KS) {
+  auto at_b = [&](int r, int c, int s) -> const T* {
+    if (MODE == 1) {
+      const int64_t n = n0 + r, k = (int64_t)s * KS + c;
+      return n < Nout && k < Kred ? We + n * Kred + k : nullptr;
+    }
+    const int64_t k = (int64_t)s * KS + r;
+    if (MODE == 2) {  // 32 gate columns, then the matching 32 up columns
+      const int64_t j = n0 + (c & 31);
+      return j < I && k < Kred ? We + k * Nout + (c < 32 ? j : I + j) : nullptr;
+    }
+    const int64_t n = n0 + c;
+    return n < Nout && k < Kred ? We + k * Nout + n : nullptr;
+  };
+  f32x16 acc;
+  mainloop<T, false, MODE != 1, VEC>(acc, (int)((Kred + KS - 1) / KS), as, bs, at_a, at_b);
+  const int rb = wm * 32 + 4 * (lane >> 5), col = lane & 31;
+  if constexpr (MODE == 2) {
+    // the up half through LDS, rows of 32 (the main loop's last barrier is behind every read)
+    if (wn == 1) {
 #pragma unroll
-    for (int u = 0; u < PT; ++u) {
-      const int i = threadIdx.x + u * 256;
-      As[i % KS][i / KS] = ra[u];
-      Bs[i / 64][i % 64] = rb[u];
+      for (int v = 0; v < 16; ++v) as[(rb + 8 * (v / 4) + v % 4) * 32 + col] = acc[v];
     }
     __syncthreads();
-    if (k0 + KS < Kred) load(k0 + KS);
+    if (wn == 1) return;
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+    for (int v = 0; v < 16; ++v) {
+      const int rr = rb + 8 * (v / 4) + v % 4;
+      const int64_t r = t.r0 + rr, j = n0 + col;
+      if (r < t.r1 && j < I) gst<T>(C, r * I + j, silu_f32(acc[v]) * as[rr * 32 + col]);
     }
-    __syncthreads();
-  }
-  if (MODE == 2) {
-    __shared__ float Cs[64][65];
+  } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) Cs[ty * 4 + i][tx * 4 + j] = acc[i][j];
-    __syncthreads();
-    for (int i = threadIdx.x; i < 64 * 32; i += 256) {
-      const int rr = i / 32, jj = i % 32;
-      const int64_t r = t.r0 + rr, j = n0 + jj;
-      if (r < t.r1 && j < I) gst<T>(C, r * I + j, silu_f32(Cs[rr][jj]) * Cs[rr][32 + jj]);
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int64_t r = t.r0 + ty * 4 + i;
-    if (r >= t.r1) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t n = n0 + tx * 4 + j;
-      if (n < Nout) gst<T>(C, r * Nout + n, acc[i][j]);
+    for (int v = 0; v < 16; ++v) {
+      const int64_t r = t.r0 + rb + 8 * (v / 4) + v % 4, n = n0 + wn * 32 + col;
+      if (r < t.r1 && n < Nout) gst<T>(C, r * Nout + n, acc[v]);
     }
   }
 }
 
-// dW[e,k,n] = sum_{r in group e} X[r,k] G[r,n]; grid (E, ceil(K/64), ceil(N/64))
-template <typename T>
-__global__ __launch_bounds__(256) void tgmm_generic_kernel(const T* __restrict__ X, const T* __restrict__ G,
-                                                           const int* __restrict__ offsets, int64_t K,
-                                                           int64_t N, T* __restrict__ dW) {
-  __shared__ float Xs[16][65];
-  __shared__ float Gs[16][65];
-  const int e = blockIdx.x;
-  const int64_t k0 = (int64_t)blockIdx.y * 64, n0 = (int64_t)blockIdx.z * 64;
+// dW[e,k,n] = sum_{r in group e} X[r,k] G[r,n]; grid (ceil(N/64), ceil(K/64), E): the tiles of the
+// largest group are dispatched first, so that its long sums do not start last
+template <typename T, int VEC>
+__global__ __launch_bounds__(NT) void tgmm_kernel(const T* __restrict__ X, const T* __restrict__ G,
+                                                  const int* __restrict__ offsets, const int* __restrict__ order,
+                                                  int64_t K, int64_t N, T* __restrict__ dW) {
+  __shared__ __attribute__((aligned(16))) float as[TILE], bs[TILE];
+  const int e = order[blockIdx.z];
+  const int64_t k0 = (int64_t)blockIdx.y * 64, n0 = (int64_t)blockIdx.x * 64;
   const int64_t r0 = offsets[e], r1 = offsets[e + 1];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-  for (int64_t rb = r0; rb < r1; rb += 16) {
-    for (int i = threadIdx.x; i < 16 * 64; i += 256) {
-      const int c = i % 64, rr = i / 64;
-      const int64_t r = rb + rr;
-      Xs[rr][c] = (r < r1 && k0 + c < K) ? gld<T>(X, r * K + k0 + c) : 0.0f;
-      Gs[rr][c] = (r < r1 && n0 + c < N) ? gld<T>(G, r * N + n0 + c) : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int rr = 0; rr < 16; ++rr) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = Xs[rr][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Gs[rr][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
+  auto at_a = [&](int r, int c, int s) -> const T* {
+    const int64_t row = r0 + (int64_t)s * KS + r, k = k0 + c;
+    return row < r1 && k < K ? X + row * K + k : nullptr;
+  };
+  auto at_b = [&](int r, int c, int s) -> const T* {
+    const int64_t row = r0 + (int64_t)s * KS + r, n = n0 + c;
+    return row < r1 && n < N ? G + row * N + n : nullptr;
+  };
+  f32x16 acc;
+  mainloop<T, true, true, VEC>(acc, (int)((r1 - r0 + KS - 1) / KS), as, bs, at_a, at_b);
+  const int lane = threadIdx.x & 63, wm = (threadIdx.x >> 6) >> 1, wn = (threadIdx.x >> 6) & 1;
   T* out = dW + (int64_t)e * K * N;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int64_t k = k0 + ty * 4 + i;
-    if (k >= K) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t n = n0 + tx * 4 + j;
-      if (n < N) gst<T>(out, k * N + n, acc[i][j]);
-    }
+  for (int v = 0; v < 16; ++v) {
+    const int64_t k = k0 + wm * 32 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4, n = n0 + wn * 32 + (lane & 31);
+    if (k < K && n < N) gst<T>(out, k * N + n, acc[v]);
   }
 }
+}  // namespace f32mm
 
 template <typename T>
 __global__ __launch_bounds__(256) void swiglu_kernel(const T* __restrict__ h, int64_t M, int64_t I,
@@ -2725,7 +2759,7 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
   if (gath) return MTX_ERR_UNSUPPORTED;
   // bf16 with widths that are multiples of 8: the 256-row MFMA tiles with partial n-tiles and
   // reduction tails.  16-byte loads and stores need aligned rows (hence the 8, and out's alignment)
-  // and the kernel's operand offsets are 32-bit.  Against the FMA kernel (6124 rows in 32 skewed
+  // and the kernel's operand offsets are 32-bit.  Against a scalar-FMA kernel (6124 rows in 32 skewed
   // groups): 1536 x 2*704 with SwiGLU 1810 -> 77 us; the smallest shapes are equal.
   if (dtype == MTX_BF16 && aligned && (uintptr_t)out % 16 == 0 && Kred > 0 && Kred % 8 == 0 && Nout % 8 == 0 &&
       out_cols % 8 == 0 && M * Kred * 2 < (int64_t(1) << 32) && Kred * Nout * 2 < (int64_t(1) << 32)) {
@@ -2748,25 +2782,31 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
     return mode == 0 ? launch_v3_edge<mf::FWD, mf::EPI_STORE>(a, grid, st)
                      : launch_v3_edge<mf::DLHS, mf::EPI_STORE>(a, grid, st);
   }
-  // generic path (exact fp32 FMA; also bf16 shapes the MFMA tiling does not cover)
+  // f32, and bf16 widths that are no multiple of 8: the f32 MFMA tiles
   rc = launch_build_tiles(gs, E, M, kMinBM, wsp, st);
   if (rc) return rc;
   const int64_t ntile_max = gmm_max_tiles(M, E, kMinBM);
   const int64_t gy = (mode == 2) ? ceil_div(I, 32) : ceil_div(Nout, 64);
   dim3 grid((unsigned)ntile_max, (unsigned)gy);
-#define MTX_GEN(T, MD)                                                                                   \
-  hipLaunchKernelGGL((gmm_generic_kernel<T, MD>), grid, dim3(256), 0, st, (const T*)x, (const T*)w, wsp.tiles, \
-                     wsp.count, Kred, Nout, (T*)out)
-  if (dtype == MTX_F32) {
-    if (mode == 0) MTX_GEN(float, 0);
-    else if (mode == 1) MTX_GEN(float, 1);
-    else MTX_GEN(float, 2);
+#define MTX_F32MM(T, MD, V)                                                                                  \
+  hipLaunchKernelGGL((f32mm::gmm_kernel<T, MD, V>), grid, dim3(f32mm::NT), 0, st, (const T*)x, (const T*)w, \
+                     wsp.tiles, wsp.count, Kred, Nout, (T*)out)
+  // 16-byte loads where every row of both operands is 16-byte aligned
+  const bool vec = aligned && Kred % 4 == 0 && Nout % 4 == 0 && (mode != 2 || I % 4 == 0);
+  if (dtype == MTX_F32 && vec) {
+    if (mode == 0) MTX_F32MM(float, 0, 4);
+    else if (mode == 1) MTX_F32MM(float, 1, 4);
+    else MTX_F32MM(float, 2, 4);
+  } else if (dtype == MTX_F32) {
+    if (mode == 0) MTX_F32MM(float, 0, 1);
+    else if (mode == 1) MTX_F32MM(float, 1, 1);
+    else MTX_F32MM(float, 2, 1);
   } else {
-    if (mode == 0) MTX_GEN(uint16_t, 0);
-    else if (mode == 1) MTX_GEN(uint16_t, 1);
-    else MTX_GEN(uint16_t, 2);
+    if (mode == 0) MTX_F32MM(uint16_t, 0, 1);
+    else if (mode == 1) MTX_F32MM(uint16_t, 1, 1);
+    else MTX_F32MM(uint16_t, 2, 1);
   }
-#undef MTX_GEN
+#undef MTX_F32MM
   return check_launch();
 }
 
@@ -2951,16 +2991,17 @@ extern "C" int mtx_tgmm(const void* x, const void* g, const int32_t* group_sizes
   if (dtype == MTX_BF16 && aligned && (uintptr_t)dw % 16 == 0 && K % 8 == 0 && N % 8 == 0 && M > 0 &&
       M * K * 2 < (int64_t(1) << 32) && M * N * 2 < (int64_t(1) << 32)) {
     // widths that are multiples of 8: partial tiles at dW's last rows and columns (6124 rows in 32
-    // skewed groups, 704 x 1536: 1994 us in the FMA kernel, 50 us here)
+    // skewed groups, 704 x 1536: 1994 us in a scalar-FMA kernel, 50 us here)
     return launch_v3_edge<mf::TGMM, mf::EPI_STORE>(tgmm_args(), E * ceil_div(K, 256) * ceil_div(N, 256), st);
   }
-  dim3 grid((unsigned)E, (unsigned)ceil_div(K, 64), (unsigned)ceil_div(N, 64));
-  if (dtype == MTX_F32)
-    hipLaunchKernelGGL(tgmm_generic_kernel<float>, grid, dim3(256), 0, st, (const float*)x, (const float*)g,
-                       wsp.offsets, K, N, (float*)dw);
-  else
-    hipLaunchKernelGGL(tgmm_generic_kernel<uint16_t>, grid, dim3(256), 0, st, (const uint16_t*)x,
-                       (const uint16_t*)g, wsp.offsets, K, N, (uint16_t*)dw);
+  dim3 grid((unsigned)ceil_div(N, 64), (unsigned)ceil_div(K, 64), (unsigned)E);
+#define MTX_F32MM(T, V)                                                                                        \
+  hipLaunchKernelGGL((f32mm::tgmm_kernel<T, V>), grid, dim3(f32mm::NT), 0, st, (const T*)x, (const T*)g, wsp.offsets, \
+                     wsp.order, K, N, (T*)dw)
+  if (dtype != MTX_F32) MTX_F32MM(uint16_t, 1);
+  else if (aligned && K % 4 == 0 && N % 4 == 0) MTX_F32MM(float, 4);
+  else MTX_F32MM(float, 1);
+#undef MTX_F32MM
   return check_launch();
 }
 
