@@ -66,15 +66,26 @@ __device__ __forceinline__ void router_select(Load load, int64_t t, bool tok_ok,
                                               float* __restrict__ scores_out, int ldo, int extra, float* smem) {
   float sel[V], pay[V];
   bool ok[V];
+  // every candidate's logit (and bias) is requested before the first is used; candidates past the
+  // end read the last expert's
+  float xs[V], bs_[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) xs[v] = load(min(li + L * v, E - 1));
+#pragma unroll
+  for (int v = 0; v < V; ++v) bs_[v] = 0.0f;
+  if (scoring == MTX_SCORING_SIGMOID_GROUP && bias) {
+#pragma unroll
+    for (int v = 0; v < V; ++v) bs_[v] = bias[min(li + L * v, E - 1)];
+  }
 #pragma unroll
   for (int v = 0; v < V; ++v) {
     const int e = li + L * v;
     ok[v] = tok_ok && e < E;
-    float x = ok[v] ? load(e) : -INFINITY;
+    const float x = ok[v] ? xs[v] : -INFINITY;
     if (scoring == MTX_SCORING_SIGMOID_GROUP) {
       const float s = 1.0f / (1.0f + expf(-x));
       pay[v] = s;
-      sel[v] = ok[v] ? s + (bias ? bias[e] : 0.0f) : -INFINITY;
+      sel[v] = ok[v] ? s + bs_[v] : -INFINITY;
     } else {
       pay[v] = x;
       sel[v] = x;
@@ -192,9 +203,11 @@ __device__ __forceinline__ void router_select(Load load, int64_t t, bool tok_ok,
   }
 }
 
-template <int V>
+// TL: logits' type (a runtime type put a branch around every load, so that each was waited for alone:
+// one token of 128 experts 8.9 us, 7.9 us with the loads together; 16 of 256 with group limits 15.5, 13.1)
+template <int V, typename TL>
 __global__ __launch_bounds__(256) void router_topk_kernel(
-    const void* __restrict__ logits, int ldt, int T, int E, int K, int L,
+    const TL* __restrict__ logits, int T, int E, int K, int L,
     int scoring, const float* __restrict__ bias, int n_group, int topk_group, int norm,
     float rscale, int32_t* __restrict__ idx_out, float* __restrict__ w_out,
     float* __restrict__ scores_out, int ldo, int extra) {
@@ -207,7 +220,12 @@ __global__ __launch_bounds__(256) void router_topk_kernel(
   const int tpb = (blockDim.x >> 6) * tpw;
   const int64_t t = (int64_t)blockIdx.x * tpb + tok_local;
   const bool tok_ok = t < T;
-  router_select<V>([&](int e) { return load_as_f32(logits, t * E + e, ldt); }, t, tok_ok, tok_local, li, L, E, K,
+  const TL* row = logits + min(t, (int64_t)T - 1) * E;
+  auto load = [&](int e) -> float {
+    if constexpr (sizeof(TL) == 4) return row[e];
+    else return bf16_to_f32(row[e]);
+  };
+  router_select<V>(load, t, tok_ok, tok_local, li, L, E, K,
                    scoring, bias, n_group, topk_group, norm, rscale, idx_out, w_out, scores_out, ldo, extra, smem);
 }
 
@@ -486,10 +504,18 @@ static int router_launch(const void* logits, int logits_dtype, int64_t T, int64_
   if (scoring == MTX_SCORING_SIGMOID_GROUP && n_group > 1 && topk_group < n_group)
     shm = (size_t)tpb * (size_t)(E + 2 * n_group) * sizeof(float);
   hipStream_t st = (hipStream_t)stream;
-#define MTX_LAUNCH_TOPK(VV)                                                                      \
-  hipLaunchKernelGGL(router_topk_kernel<VV>, dim3(grid), dim3(256), shm, st, logits, logits_dtype, \
-                     (int)T, (int)E, (int)K, L, scoring, bias, (int)n_group, (int)topk_group,      \
-                     norm_topk_prob, routed_scaling_factor, topk_idx, topk_w, scores, (int)ldo, (int)extra)
+#define MTX_LAUNCH_TOPK(VV)                                                                                  \
+  do {                                                                                                       \
+    if (logits_dtype == MTX_F32)                                                                             \
+      hipLaunchKernelGGL((router_topk_kernel<VV, float>), dim3(grid), dim3(256), shm, st, (const float*)logits, \
+                         (int)T, (int)E, (int)K, L, scoring, bias, (int)n_group, (int)topk_group,            \
+                         norm_topk_prob, routed_scaling_factor, topk_idx, topk_w, scores, (int)ldo, (int)extra); \
+    else                                                                                                     \
+      hipLaunchKernelGGL((router_topk_kernel<VV, uint16_t>), dim3(grid), dim3(256), shm, st,                 \
+                         (const uint16_t*)logits, (int)T, (int)E, (int)K, L, scoring, bias, (int)n_group,    \
+                         (int)topk_group, norm_topk_prob, routed_scaling_factor, topk_idx, topk_w, scores,   \
+                         (int)ldo, (int)extra);                                                              \
+  } while (0)
   if (V <= 1) MTX_LAUNCH_TOPK(1);
   else if (V <= 2) MTX_LAUNCH_TOPK(2);
   else if (V <= 4) MTX_LAUNCH_TOPK(4);
