@@ -382,6 +382,29 @@ int mtx_tgmm_fp8_p2(const uint8_t* xt, const float* xt_scale, const uint8_t* gt,
                     const int32_t* group_sizes, int64_t M, int64_t F, int64_t N, int64_t E, void* dw,
                     void* workspace, int64_t workspace_bytes, void* stream);
 
+/* A training step's operands, quantised where they are made (no counterpart; the codes and scales are
+ * those of the calls above, p2 != 0 for the power-of-two mode).
+ * mtx_quant_fp8_weights_both: mtx_quant_fp8_weights and mtx_quant_fp8_weights_t from one read of w.
+ * mtx_fp8_chunks: the expert chunks of group_sizes, into a workspace of
+ *   mtx_fp8_grouped_workspace_size(E) bytes that mtx_quant_fp8_operands takes as `chunks`.
+ * mtx_quant_fp8_operands: a bf16 matrix X [M, F] of expert-sorted rows, quantised in 1x128 row groups
+ *   (row_q, row_scale as mtx_quant_fp8_rows; both may be NULL) and in 128-row chunks, transposed
+ *   (xt, xt_scale as mtx_quant_fp8_grouped_t with the same `blocks`; both may be NULL).  source:
+ *   0: X = a [M, F];  1: X[r] = a[row_index[r] / index_div] (a [a_rows, F], indices clamped);
+ *   2: X = SwiGLU of a [M, 2F], rounded to bf16.  Rows past sum(group_sizes) get no codes.
+ * mtx_gmm_fp8_gathered: mtx_gmm_fp8 on rows row_index[r] / index_div of xq / x_scale (x_rows rows). */
+int mtx_quant_fp8_weights_both(const void* w, int dtype, int64_t E, int64_t Kin, int64_t Kout, int p2,
+                               uint8_t* w_q, float* w_scale, uint8_t* w_qt, float* w_scale_t, void* stream);
+int mtx_fp8_chunks(const int32_t* group_sizes, int64_t M, int64_t E, void* workspace, int64_t workspace_bytes,
+                   void* stream);
+int mtx_quant_fp8_operands(int source, const void* a, const int32_t* row_index, int64_t index_div,
+                           int64_t a_rows, int64_t M, int64_t F, int64_t E, int blocks, int p2, uint8_t* row_q,
+                           float* row_scale, uint8_t* xt, float* xt_scale, const void* chunks, void* stream);
+int mtx_gmm_fp8_gathered(const uint8_t* xq, const float* x_scale, int64_t x_rows, const int32_t* row_index,
+                         int64_t index_div, const uint8_t* w_q, const float* w_scale, const int32_t* group_sizes,
+                         int64_t M, int64_t Kin, int64_t Kout, int64_t E, int p2, void* out, void* workspace,
+                         int64_t workspace_bytes, void* stream);
+
 /* ---- expert weight layouts -------------------------------------------------------------
  * Batched transpose-copy (the per-expert HF <-> fused conversions of
  * mintext/checkpoint/conversion.py:80-166, done on the device at load time):

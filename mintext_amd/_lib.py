@@ -86,6 +86,10 @@ SIGNATURES = {
     "mtx_gmm_fp8_dlhs_p2": (_I, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _I64, _P]),
     "mtx_quant_fp8_grouped_t_p2": (_I, [_P, _I, _P, _I64, _I64, _I64, _I, _P, _P, _P, _I64, _P]),
     "mtx_tgmm_fp8_p2": (_I, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _I64, _P]),
+    "mtx_gmm_fp8_gathered": (_I, [_P, _P, _I64, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _P, _I64, _P]),
+    "mtx_quant_fp8_weights_both": (_I, [_P, _I, _I64, _I64, _I64, _I, _P, _P, _P, _P, _P]),
+    "mtx_fp8_chunks": (_I, [_P, _I64, _I64, _P, _I64, _P]),
+    "mtx_quant_fp8_operands": (_I, [_I, _P, _P, _I64, _I64, _I64, _I64, _I64, _I, _I, _P, _P, _P, _P, _P, _P]),
     "mtx_transpose_batched": (_I, [_P, _I, _I64, _I64, _I64, _I64, _I64, _P, _I64, _I64, _P]),
     "mtx_stream_copy": (_I, [_P, _P, _I64, _I, _I64, _P]),
 }

@@ -1385,13 +1385,20 @@ static int fp8_checks(const void* xq, const float* xs, const uint8_t* wq, const 
 
 static int gmm_fp8_entry(bool p2, const uint8_t* xq, const float* x_scale, const uint8_t* w_q, const float* w_scale,
                          const int32_t* group_sizes, int64_t M, int64_t Kin, int64_t Kout, int64_t E, void* out,
-                         void* workspace, int64_t workspace_bytes, void* stream) {
+                         void* workspace, int64_t workspace_bytes, void* stream, const int32_t* gather = nullptr,
+                         int64_t gather_div = 1, int64_t gather_rows = 0) {
   int rc = fp8_checks(xq, x_scale, w_q, w_scale, group_sizes, M, Kin, E, workspace, workspace_bytes);
   if (rc) return rc;
   if (Kout <= 0 || Kout % 256) return (Kout % 128 == 0 && Kout > 0) ? MTX_ERR_UNSUPPORTED : MTX_ERR_ARG;
+  if (gather && (gather_div < 1 || gather_div > INT32_MAX || gather_rows < 0 || gather_rows > INT32_MAX / 2 ||
+                 (gather_rows == 0 && M > 0)))
+    return MTX_ERR_ARG;
   if (M == 0) return MTX_OK;
   if (!out) return MTX_ERR_ARG;
   f8::Args a{};
+  a.gather = gather;
+  a.gather_div = (int)gather_div;
+  a.gather_rows = (int)gather_rows;
   a.xq = xq;
   a.xs = x_scale;
   a.wq = w_q;
@@ -1418,6 +1425,15 @@ extern "C" int mtx_gmm_fp8_p2(const uint8_t* xq, const float* x_scale, const uin
                               void* workspace, int64_t workspace_bytes, void* stream) {
   return gmm_fp8_entry(true, xq, x_scale, w_q, w_scale, group_sizes, M, Kin, Kout, E, out, workspace,
                        workspace_bytes, stream);
+}
+
+extern "C" int mtx_gmm_fp8_gathered(const uint8_t* xq, const float* x_scale, int64_t x_rows, const int32_t* row_index,
+                                    int64_t index_div, const uint8_t* w_q, const float* w_scale,
+                                    const int32_t* group_sizes, int64_t M, int64_t Kin, int64_t Kout, int64_t E, int p2,
+                                    void* out, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!row_index && M > 0) return MTX_ERR_ARG;
+  return gmm_fp8_entry(p2 != 0, xq, x_scale, w_q, w_scale, group_sizes, M, Kin, Kout, E, out, workspace, workspace_bytes,
+                       stream, row_index, index_div, x_rows);
 }
 
 static int fp8_swiglu_entry(const uint8_t* xq, const float* x_scale, const uint8_t* w_q, const float* w_scale,

@@ -56,6 +56,36 @@ __global__ __launch_bounds__(256) void quant_weights_t_kernel(const T* __restric
   if (threadIdx.x == 0) ws[(e * (Kin / 128) + blockIdx.y) * (Kout / 128) + blockIdx.x] = s;
 }
 
+// Both forms of the weight codes from one read: the forward's transposed ones (quant_weights_kernel)
+// and W's own layout (above) hold the same codes under the same block scales.  A training step
+// needs both; HBM-bound, 4 bytes per bf16 element instead of 6.
+template <typename T, bool P2>
+__global__ __launch_bounds__(256) void quant_weights_both_kernel(const T* __restrict__ w, int64_t Kin, int64_t Kout,
+                                                                 uint8_t* __restrict__ wq, float* __restrict__ ws,
+                                                                 uint8_t* __restrict__ wqt, float* __restrict__ wst) {
+  __shared__ __attribute__((aligned(16))) uint8_t tt[128 * q8::TSTRIDE];
+  __shared__ float red[4];
+  using S = q8::TileShape<T>;
+  const int64_t e = blockIdx.z, k0 = (int64_t)blockIdx.y * 128, n0 = (int64_t)blockIdx.x * 128;
+  const int64_t base = (e * Kin + k0) * Kout + n0;
+  q8::Tile<T> t;
+  t.load(w + base, Kout, 128);
+  float m[S::VE];
+  t.col_amax(m);
+  float a = 0.0f;
+#pragma unroll
+  for (int j = 0; j < S::VE; ++j) a = fmaxf(a, m[j]);
+  const float s = q8::block_scale<P2>(a, red);
+  q8::codes_to_lds_t(t, [&](int) { return s; }, tt);
+  q8::codes_to_global(t, s, wqt + base, Kout);
+  __syncthreads();
+  q8::lds_t_to_global(tt, wq + (e * Kout + n0) * Kin + k0, Kin);
+  if (threadIdx.x == 0) {
+    wst[(e * (Kin / 128) + blockIdx.y) * (Kout / 128) + blockIdx.x] = s;
+    ws[(e * (Kout / 128) + blockIdx.x) * (Kin / 128) + blockIdx.y] = s;
+  }
+}
+
 // ---- expert chunks -----------------------------------------------------------------------------
 // One workgroup, E <= 1024: row offsets off[E+1] of the groups (clamped to M like the forward's
 // tile builder), chunk bases cb[E+1] (cb[e] = sum of ceil(rows/128) over the experts before e)
@@ -176,6 +206,149 @@ __global__ __launch_bounds__(256) void quant_grouped_t_kernel(const T* __restric
   __syncthreads();
   const int64_t lde = (int64_t)128 * ne;
   q8::lds_t_to_global(tt, xt + (int64_t)128 * F * cb[e] + (int64_t)128 * j + f0 * lde, lde);
+}
+
+// ---- a training step's operands, quantised where they are made -------------------------------------
+// One workgroup makes a 128-row x 128-feature bf16 tile of an expert's chunk and quantises it both
+// ways: 1x128 along its rows (the operand of a forward or dlhs product; rq [M, F], rs [M, F/128]) and
+// along the chunk's rows, transposed (the tgmm operand of quant_grouped_t_kernel, same layout).  Codes
+// and scales are those of the separate kernels.  Where the tile comes from:
+//   ROWS    x [M, F] itself;
+//   GATHER  sorted row r is token row_index[r] / div of a [src_rows, F] (the dispatch copy is never
+//           written; only the transposed codes, the row codes being taken per token);
+//   SWIGLU  silu(gate) * up of h [M, 2F], rounded to bf16 as mtx_swiglu does.
+// HBM-bound (4.9-5.2 TB/s; SWIGLU about as much by its exp and division).  65536 rows in 64 groups: ROWS
+// of 2048 features 104 us (71 + 94 apart), GATHER 67 us (dispatch 49 + 97), SWIGLU of 768 features 90 us
+// (54 + 27 + 38).  A chunk's feature blocks run side by side, so that whole rows are read together:
+// with a feature's chunks side by side ROWS took 124 us and GATHER 76.  The SwiGLU VJP as a source held
+// both of its tiles in 187 registers and ran at two waves per SIMD: 190 us against 160 for
+// mtx_swiglu_bwd and ROWS.  Rows of no group are not written (the products never use them).
+enum { Q_ROWS = 0, Q_GATHER = 1, Q_SWIGLU = 2 };
+struct QArgs {
+  const uint16_t* a;
+  const int32_t* row_index;  // GATHER
+  int div, src_rows;
+  int F, E, nfb;             // nfb: F / 128
+  const int* cb;
+  const int* off;
+  uint8_t* rq;               // nullptr: no row codes
+  float* rs;
+  uint8_t* xt;               // nullptr: no transposed codes
+  float* xts;
+};
+template <int SRC, bool BLOCK, bool P2>
+__global__ __launch_bounds__(256) void quant_operands_kernel(QArgs p) {
+  using S = q8::TileShape<uint16_t>;
+  static_assert(S::VE == 8 && S::LPR == 16, "16 lanes of 8 bf16 hold a tile row");
+  __shared__ __attribute__((aligned(16))) uint8_t tt[128 * q8::TSTRIDE];
+  __shared__ float red[S::TR][128];
+  __shared__ float scs[128];
+  const int c = blockIdx.x / p.nfb, fb = blockIdx.x % p.nfb, tid = threadIdx.x;
+  if (c >= p.cb[p.E]) return;  // beyond the chunks of this call's groups
+  const int e = chunk_expert(p.cb, p.E, c);
+  const int j = c - p.cb[e], ne = p.cb[e + 1] - p.cb[e];
+  const int r0 = p.off[e] + 128 * j, nr = min(128, p.off[e + 1] - r0);
+  q8::Tile<uint16_t> t;
+  t.cl = tid % S::LPR;
+  t.rl = tid / S::LPR;
+  auto row_of = [&](int h, int q) { return 4 * (t.rl + S::TR * h) + q; };
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+
+  const int64_t f0 = (int64_t)fb * 128, col = f0 + t.cl * 8;
+  if constexpr (SRC == Q_ROWS || SRC == Q_GATHER) {
+#pragma unroll
+    for (int h = 0; h < S::G4; ++h)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = row_of(h, q);
+        int64_t src = r0 + min(r, nr - 1);
+        if (SRC == Q_GATHER) src = min(max(p.row_index[src], 0) / p.div, p.src_rows - 1);
+        const u32x4 v = *(const u32x4*)(p.a + src * p.F + col);
+        t.raw[h][q] = r < nr ? v : zero;
+      }
+  } else {
+    // h rows hold the gate half, then the up half, F columns each
+    auto el = [](const u32x4& v, int i) {
+      return __uint_as_float((i & 1) ? (v[i >> 1] & 0xffff0000u) : (v[i >> 1] << 16));
+    };
+#pragma unroll
+    for (int h = 0; h < S::G4; ++h) {
+      u32x4 g[4], u[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t src = r0 + min(row_of(h, q), nr - 1);
+        g[q] = *(const u32x4*)(p.a + src * 2 * p.F + col);
+        u[q] = *(const u32x4*)(p.a + src * 2 * p.F + p.F + col);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        u32x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          o[i] = pack_bf16x2(silu_f32(el(g[q], 2 * i)) * el(u[q], 2 * i),
+                             silu_f32(el(g[q], 2 * i + 1)) * el(u[q], 2 * i + 1));
+        t.raw[h][q] = row_of(h, q) < nr ? o : zero;
+      }
+    }
+  }
+  if (p.rq) {
+#pragma unroll
+    for (int h = 0; h < S::G4; ++h)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(t.at(h, q, i)));
+        m = max8_lanes(m);
+        m = fmaxf(m, lane_xchg<3>(m));
+        const float s = q8::scale_of<P2>(m);
+        const int r = row_of(h, q);
+        if (r >= nr) continue;
+        const float rs = 1.0f / s;
+        float v[8];
+        if constexpr (P2) {  // the exact quotient by a power of two
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[i] = t.at(h, q, i) * rs;
+        } else if (__builtin_expect(div_rn_ok(s), 1)) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[i] = div_rn(t.at(h, q, i), s, rs);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[i] = t.at(h, q, i) / s;
+        }
+        *(q8::u32x2*)(p.rq + (int64_t)(r0 + r) * p.F + f0 + t.cl * 8) =
+            q8::u32x2{e4m3_pack4(v[0], v[1], v[2], v[3]), e4m3_pack4(v[4], v[5], v[6], v[7])};
+        if (t.cl == 0) p.rs[(int64_t)(r0 + r) * (p.F / 128) + fb] = s;
+      }
+  }
+  if (!p.xt) return;
+  float m[8];
+  t.col_amax(m);
+  if (BLOCK) {
+    float a = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a = fmaxf(a, m[i]);
+    const float s = q8::block_scale<P2>(a, &red[0][0]);
+    q8::codes_to_lds_t<P2>(t, [&](int) { return s; }, tt);
+    if (tid == 0) p.xts[(int64_t)(p.F / 128) * p.cb[e] + (int64_t)fb * ne + j] = s;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) red[t.rl][t.cl * 8 + i] = m[i];
+    __syncthreads();
+    if (tid < 128) {
+      float a = 0.0f;
+#pragma unroll
+      for (int r = 0; r < S::TR; ++r) a = fmaxf(a, red[r][tid]);
+      const float s = q8::scale_of<P2>(a);
+      scs[tid] = s;
+      p.xts[(int64_t)p.F * p.cb[e] + (f0 + tid) * ne + j] = s;
+    }
+    __syncthreads();
+    q8::codes_to_lds_t<P2>(t, [&](int i) { return scs[t.cl * 8 + i]; }, tt);
+  }
+  __syncthreads();
+  const int64_t lde = (int64_t)128 * ne;
+  q8::lds_t_to_global(tt, p.xt + (int64_t)128 * p.F * p.cb[e] + (int64_t)128 * j + f0 * lde, lde);
 }
 
 // ---- tgmm: dW[e] = XT_e GT_e^T over the expert's chunks ---------------------------------------------
@@ -886,6 +1059,85 @@ extern "C" int mtx_quant_fp8_grouped_t_p2(const void* x, int dtype, const int32_
                                           int64_t workspace_bytes, void* stream) {
   return quant_grouped_t_entry<true>(x, dtype, group_sizes, M, F, E, blocks, xt, xt_scale, workspace,
                                      workspace_bytes, stream);
+}
+
+extern "C" int mtx_quant_fp8_weights_both(const void* w, int dtype, int64_t E, int64_t Kin, int64_t Kout, int p2,
+                                          uint8_t* w_q, float* w_scale, uint8_t* w_qt, float* w_scale_t, void* stream) {
+  if (E < 0 || Kin < 0 || Kout < 0 || Kin % 128 || Kout % 128 || (dtype != MTX_F32 && dtype != MTX_BF16))
+    return MTX_ERR_ARG;
+  if (E == 0 || Kin == 0 || Kout == 0) return MTX_OK;
+  if (!w || !w_q || !w_scale || !w_qt || !w_scale_t) return MTX_ERR_ARG;
+  if (((uintptr_t)w | (uintptr_t)w_q | (uintptr_t)w_qt) % 16) return MTX_ERR_ARG;
+  if (E > 65535 || Kin / 128 > 65535) return MTX_ERR_UNSUPPORTED;
+  dim3 grid((unsigned)(Kout / 128), (unsigned)(Kin / 128), (unsigned)E);
+  hipStream_t st = (hipStream_t)stream;
+#define MTX_QB(T, P)                                                                                                 \
+  hipLaunchKernelGGL((f8b::quant_weights_both_kernel<T, P>), grid, dim3(256), 0, st, (const T*)w, Kin, Kout, w_q, w_scale, \
+                     w_qt, w_scale_t)
+  if (dtype == MTX_F32) {
+    if (p2) MTX_QB(float, true);
+    else MTX_QB(float, false);
+  } else {
+    if (p2) MTX_QB(uint16_t, true);
+    else MTX_QB(uint16_t, false);
+  }
+#undef MTX_QB
+  return check_launch();
+}
+
+extern "C" int mtx_fp8_chunks(const int32_t* group_sizes, int64_t M, int64_t E, void* workspace,
+                              int64_t workspace_bytes, void* stream) {
+  if (M < 0 || M > INT32_MAX / 2 || E < 1 || E > 1024) return MTX_ERR_ARG;
+  if (!workspace || workspace_bytes < mtx_fp8_grouped_workspace_size(E)) return MTX_ERR_WORKSPACE;
+  if (!group_sizes) return MTX_ERR_ARG;
+  int *cb, *off, *order;
+  return grouped_prologue(group_sizes, E, M, workspace, (hipStream_t)stream, &cb, &off, &order);
+}
+
+extern "C" int mtx_quant_fp8_operands(int source, const void* a, const int32_t* row_index,
+                                      int64_t index_div, int64_t a_rows, int64_t M, int64_t F, int64_t E, int blocks,
+                                      int p2, uint8_t* row_q, float* row_scale, uint8_t* xt, float* xt_scale,
+                                      const void* chunks, void* stream) {
+  if (source < f8b::Q_ROWS || source > f8b::Q_SWIGLU) return MTX_ERR_ARG;
+  if (M < 0 || M > INT32_MAX / 2 || F <= 0 || F % 128 || E < 1 || E > 1024)
+    return MTX_ERR_ARG;
+  if (M == 0) return MTX_OK;
+  if (!a || !chunks) return MTX_ERR_ARG;
+  if ((row_q != nullptr) != (row_scale != nullptr) || (xt != nullptr) != (xt_scale != nullptr)) return MTX_ERR_ARG;
+  if (source == f8b::Q_GATHER &&
+      (!row_index || index_div < 1 || index_div > INT32_MAX || a_rows < 1 || a_rows > INT32_MAX / 2))
+    return MTX_ERR_ARG;
+  if (((uintptr_t)a | (uintptr_t)row_q | (uintptr_t)xt) % 16) return MTX_ERR_ARG;
+  const int64_t C = fp8_grouped_chunks(M, E), fb = F / 128;
+  if (C > 2147483647 / 128 || C * fb > INT32_MAX) return MTX_ERR_UNSUPPORTED;
+  f8b::QArgs q{};
+  q.a = (const uint16_t*)a;
+  q.row_index = row_index;
+  q.div = (int)index_div;
+  q.src_rows = (int)a_rows;
+  q.F = (int)F;
+  q.E = (int)E;
+  q.cb = (const int*)chunks;
+  q.off = q.cb + E + 1;
+  q.rq = row_q;
+  q.rs = row_scale;
+  q.xt = xt;
+  q.xts = xt_scale;
+  q.nfb = (int)fb;
+  const dim3 grid((unsigned)(C * fb));
+  hipStream_t st = (hipStream_t)stream;
+#define MTX_QO(SRC)                                                                                                \
+  do {                                                                                                             \
+    if (blocks && p2) hipLaunchKernelGGL((f8b::quant_operands_kernel<SRC, true, true>), grid, dim3(256), 0, st, q); \
+    else if (blocks) hipLaunchKernelGGL((f8b::quant_operands_kernel<SRC, true, false>), grid, dim3(256), 0, st, q); \
+    else if (p2) hipLaunchKernelGGL((f8b::quant_operands_kernel<SRC, false, true>), grid, dim3(256), 0, st, q);    \
+    else hipLaunchKernelGGL((f8b::quant_operands_kernel<SRC, false, false>), grid, dim3(256), 0, st, q);           \
+  } while (0)
+  if (source == f8b::Q_ROWS) MTX_QO(f8b::Q_ROWS);
+  else if (source == f8b::Q_GATHER) MTX_QO(f8b::Q_GATHER);
+  else MTX_QO(f8b::Q_SWIGLU);
+#undef MTX_QO
+  return check_launch();
 }
 
 static int tgmm_fp8_entry(bool p2, const uint8_t* xt, const float* xt_scale, const uint8_t* gt,

@@ -88,7 +88,8 @@ __device__ __forceinline__ float block_scale(float m, float* red) {
 // Codes of the tile transposed into LDS: tt[c * TSTRIDE + r] = code of (row r, column c), written as
 // one 32-bit word per (column, group of four rows).  sc(j) is the scale of column cl*VE + j.
 constexpr int TSTRIDE = 132;  // bytes per transposed row: 4-byte aligned, 2-way bank spread
-template <typename T, typename SC>
+// P2: the scales are powers of two, whose quotient is the product with the (exact) reciprocal.
+template <bool P2 = false, typename T, typename SC>
 __device__ __forceinline__ void codes_to_lds_t(const Tile<T>& t, SC sc, uint8_t* tt) {
   using S = TileShape<T>;
   auto put = [&](auto quot) {
@@ -110,7 +111,8 @@ __device__ __forceinline__ void codes_to_lds_t(const Tile<T>& t, SC sc, uint8_t*
     fast = fast && div_rn_ok(sc(j));
     rs[j] = 1.0f / sc(j);
   }
-  if (__builtin_expect(fast, 1)) put([&](float a, int j) { return div_rn(a, sc(j), rs[j]); });
+  if constexpr (P2) put([&](float a, int j) { return a * rs[j]; });
+  else if (__builtin_expect(fast, 1)) put([&](float a, int j) { return div_rn(a, sc(j), rs[j]); });
   else put([&](float a, int j) { return a / sc(j); });
 }
 

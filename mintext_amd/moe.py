@@ -241,7 +241,11 @@ def moe_experts_forward_fp8_train(x: torch.Tensor, topk_indices: torch.Tensor, t
     Gradients reach x, topk_weights, gate_up and down.  ``scales``: "amax" (amax / 448) or "pow2"
     (power-of-two scales applied by the MFMA) in every quantisation."""
     from .kernels.fp8 import grouped_matmul_fp8_vjp
+    from .kernels.fp8_train import experts_fp8_train, experts_fp8_train_supported
 
+    if experts_fp8_train_supported(x, topk_indices, topk_weights, gate_up, down, scales):
+        # the steps below as one autograd node, its quantisers fused with what makes their operands
+        return experts_fp8_train(x, topk_indices, topk_weights, gate_up, down, scales)
     E = gate_up.shape[0]
     sorted_tokens, sort_indices, group_sizes = route(x, topk_indices, E)
     h = grouped_matmul_fp8_vjp(sorted_tokens, gate_up, group_sizes, scales=scales)
