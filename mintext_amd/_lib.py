@@ -127,11 +127,17 @@ def call(name: str, *args) -> None:
         raise MtxError(name, rc, detail)
 
 
-def query(name: str, *args) -> int:
-    v = getattr(lib(), name)(*args)
+@functools.lru_cache(maxsize=4096)
+def _query(handle, name: str, *args) -> int:
+    v = getattr(handle, name)(*args)
     if v < 0:
         raise MtxError(name, int(v), "invalid sizes")
     return int(v)
+
+
+def query(name: str, *args) -> int:
+    """A size that depends on the arguments alone (``*_workspace_size``, ``mtx_fp8_grouped_chunks``)."""
+    return _query(lib(), name, *args)
 
 
 def dtype_code(dt: torch.dtype) -> int:
@@ -167,7 +173,17 @@ def require_device(*tensors) -> torch.device:
 
 
 def stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """Handle of the current stream of ``device`` (a tensor's, so with an index); asked for on each call,
+    without building a Stream object."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+def plain_forward(*tensors) -> bool:
+    """Whether an autograd Function's forward can run without the Function: no gradient is asked for, and
+    no forward-mode level or functorch transform is active that would have to see (and refuse) it."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    return torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:

@@ -168,7 +168,14 @@ def grouped_matmul(x: torch.Tensor, weights: torch.Tensor, group_sizes: torch.Te
     Returns:
         [M, K_out] in x's dtype.
     """
-    return _GMM.apply(x, weights, group_sizes, None if tiling is None else _pad_tiling(tiling))
+    return _grouped_matmul(x, weights, group_sizes, tiling)
+
+
+def _grouped_matmul(x, weights, group_sizes, tiling):
+    tiling9 = None if tiling is None else _pad_tiling(tiling)
+    if L.plain_forward(x, weights):
+        return _gmm_fwd(x, weights, _gs(group_sizes), None if tiling9 is None else tiling9[0:3])
+    return _GMM.apply(x, weights, group_sizes, tiling9)
 
 
 def grouped_matmul_vjp(x: torch.Tensor, weights: torch.Tensor, group_sizes: torch.Tensor, *,
@@ -182,7 +189,7 @@ def grouped_matmul_vjp(x: torch.Tensor, weights: torch.Tensor, group_sizes: torc
     ``mosaic_fusion`` is accepted and ignored.
     """
     del mosaic_fusion
-    return _GMM.apply(x, weights, group_sizes, None if tiling is None else _pad_tiling(tiling))
+    return _grouped_matmul(x, weights, group_sizes, tiling)
 
 
 def grouped_matmul_swiglu(x: torch.Tensor, weights: torch.Tensor, group_sizes: torch.Tensor, *,

@@ -96,6 +96,7 @@ def _combine(Y: torch.Tensor, inv: torch.Tensor, w: torch.Tensor | None, N: int,
 class _Route(torch.autograd.Function):
     @staticmethod
     def forward(ctx, tokens, topk_indices, num_experts):
+        ctx.set_materialize_grads(False)  # no zero fills for the whole-number outputs
         sorted_tokens, sort_indices, group_sizes, inverse = _route_impl(tokens, topk_indices, num_experts)
         ctx.save_for_backward(inverse)
         ctx.nk = topk_indices.shape
@@ -107,6 +108,8 @@ class _Route(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_sorted, _g_si, _g_gs):
+        if g_sorted is None:
+            return None, None, None
         (inverse,) = ctx.saved_tensors
         N, K = ctx.nk
         # d tokens[n] = sum_k d sorted[inverse[n*K+k]]  (repeat VJP after the sort VJP)
@@ -131,22 +134,27 @@ def _combine_add(Y: torch.Tensor, inv: torch.Tensor, w: torch.Tensor, N: int, K:
     return out
 
 
+def _unroute_forward(sorted_output, sort_indices, topk_weights, K, addend=None):
+    """(unroute [+ addend], inverse permutation, contiguous weights)"""
+    N = topk_weights.shape[0]
+    inv = _inverse_of(sort_indices)
+    out_dtype = torch.result_type(sorted_output, topk_weights)
+    if out_dtype not in (torch.float32, torch.bfloat16):
+        raise TypeError(f"unroute output dtype {out_dtype} not supported")
+    w = topk_weights.contiguous()
+    if addend is None:
+        return _combine(sorted_output, inv, w, N, K, out_dtype), inv, w
+    return _combine_add(sorted_output, inv, w, N, K, addend, out_dtype), inv, w
+
+
 class _Unroute(torch.autograd.Function):
     """unroute, and with an addend unroute + addend (one combine pass either way); the VJP is
     ``mtx_unroute_bwd`` for the expert outputs and weights, the identity for the addend."""
 
     @staticmethod
     def forward(ctx, sorted_output, sort_indices, topk_weights, K, addend=None):
-        N = topk_weights.shape[0]
-        inv = _inverse_of(sort_indices)
-        out_dtype = torch.result_type(sorted_output, topk_weights)
-        if out_dtype not in (torch.float32, torch.bfloat16):
-            raise TypeError(f"unroute output dtype {out_dtype} not supported")
-        w = topk_weights.contiguous()
-        if addend is None:
-            out = _combine(sorted_output, inv, w, N, K, out_dtype)
-        else:
-            out = _combine_add(sorted_output, inv, w, N, K, addend, out_dtype)
+        out, inv, w = _unroute_forward(sorted_output, sort_indices, topk_weights, K, addend)
+        if addend is not None:
             ctx.add_dtype = addend.dtype
         ctx.save_for_backward(sorted_output, inv, w)
         ctx.K = K
@@ -223,6 +231,11 @@ def route(tokens: torch.Tensor, topk_indices: torch.Tensor, num_experts: int):
     """
     if tokens.dtype == torch.float8_e4m3fn:
         return _route_impl(tokens, topk_indices, num_experts)[:3]
+    if L.plain_forward(tokens):
+        sorted_tokens, sort_indices, group_sizes, inverse = _route_impl(tokens, topk_indices, int(num_experts))
+        sort_indices._mtx_inverse = inverse
+        sort_indices._mtx_version = sort_indices._version
+        return sorted_tokens, sort_indices, group_sizes
     return _Route.apply(tokens, topk_indices, int(num_experts))
 
 
@@ -232,6 +245,8 @@ def unroute(sorted_output: torch.Tensor, sort_indices: torch.Tensor, topk_weight
 
     Returns [N, D] in ``result_type(sorted_output, topk_weights)``.
     """
+    if L.plain_forward(sorted_output, topk_weights):
+        return _unroute_forward(sorted_output, sort_indices, topk_weights, int(num_experts_per_tok))[0]
     return _Unroute.apply(sorted_output, sort_indices, topk_weights, int(num_experts_per_tok))
 
 
@@ -242,6 +257,8 @@ def unroute_add(sorted_output: torch.Tensor, sort_indices: torch.Tensor, topk_we
     (``mtx_unroute_add``; the same f32 bits as the two steps).  ``addend`` is [N, D] float32 or
     bfloat16.  Differentiable in the expert outputs, the weights and the addend.
     """
+    if L.plain_forward(sorted_output, topk_weights, addend):
+        return _unroute_forward(sorted_output, sort_indices, topk_weights, int(num_experts_per_tok), addend)[0]
     return _Unroute.apply(sorted_output, sort_indices, topk_weights, int(num_experts_per_tok), addend)
 
 

@@ -70,6 +70,7 @@ class _RouterTopK(torch.autograd.Function):
     def forward(ctx, lg, k, scoring, b, n_group, topk_group, norm, rscale, return_scores, shared_expert):
         idx, w, scores = _router_fwd(lg, k, scoring, b, n_group, topk_group, norm, rscale, return_scores,
                                      shared_expert)
+        ctx.set_materialize_grads(False)  # no zero fill for the indices
         ctx.mark_non_differentiable(idx)
         ctx.save_for_backward(lg, idx)
         ctx.cfg = (k, scoring, norm, rscale)
