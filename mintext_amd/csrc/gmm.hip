@@ -2507,15 +2507,22 @@ static int launch_v3_edge(const mf::Args& a, int64_t grid, hipStream_t st) {
   hipLaunchKernelGGL((mf::gmm_v3_kernel<MODE, EPI, 2, 4, 256, 4, true>), dim3((unsigned)grid), dim3(512), 0, st, a);
   return check_launch();
 }
-// Persistent plain-store kernel for reductions of 4 .. MTX_V4P_MAX_STAGES 32-k stages (0: never):
-// one workgroup per CU, each walking its XCD's share of the tile list.  Measured against
-// gmm_v3_kernel on the same box (E = 8, M = 16384, N = 4096): +36 % at Kred 512, +10 % at 1024,
-// but -8 % at 2048 and -26 % at 4096, and -10 % / -19 % on the C5 dlhs / C3 down shapes (Kred
-// 1536-2048).  vmcnt counts loads and stores in one in-order counter, so the next tile's first
-// ring wait also waits for the previous tile's epilogue stores, which a short-lived v3 workgroup
-// leaves draining behind it; that costs more than the saved ring fill once tiles are long.
+// Persistent plain-store kernel for reductions of 4 .. MTX_V4P_MAX_STAGES 32-k stages and groups of at
+// least MTX_V4P_MIN_MEAN rows on average: one workgroup per CU, each walking its XCD's share of the
+// tile list.  Against gmm_v3_kernel (us, this / v3): 16384 rows in 8 groups, Kred 512 x 4096 102 / 106,
+// 1024 x 4096 168 / 170, 256 x 2048 43 / 45.  Smaller groups leave partly empty last m-tiles and few
+// tiles per workgroup, which its static shares cannot even out: 8192 rows in 8 groups, 1024 x 4096
+// 123 / 99; 32 groups of 512 rows, 768 x 2048 93 / 85; 128 groups of 256, 768 x 2048 185 / 168 (Zipf
+// loads 217 / 178), of 128 148 / 111.  (gmm_w4_kernel loses to v3 on short reductions: 53 / 39 for 8192
+// rows in 8 groups, 512 x 2048; 101 / 85 for the 32 groups.)  On longer reductions it lost 8 % at Kred
+// 2048 and 26 % at 4096: vmcnt counts loads and stores in one in-order counter, so the next tile's
+// first ring wait also waits for the previous tile's epilogue stores, which a short-lived v3
+// workgroup leaves draining behind it; that costs more than the saved ring fill once tiles are long.
 #ifndef MTX_V4P_MAX_STAGES
 #define MTX_V4P_MAX_STAGES 32
+#endif
+#ifndef MTX_V4P_MIN_MEAN
+#define MTX_V4P_MIN_MEAN 2048
 #endif
 template <int MODE>
 static int launch_v4p(const mf::Args& a, int64_t max_tiles, int ncu, hipStream_t st) {
@@ -2681,7 +2688,8 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
       return MTX_ERR_UNSUPPORTED;
     // one m-tile per scheduling group: spread the m-tiles of experts with several of them
     const int spread = (a.gm == 1) ? MTX_SPREAD_MIN : 0;
-    const bool w4 = big_m && (M / E) >= MTX_W4_MIN_MEAN;
+    const bool short_k = mode != 2 && Kred <= MTX_V4P_MAX_STAGES * mf::v3::BKS;  // plain stores only
+    const bool w4 = big_m && (M / E) >= MTX_W4_MIN_MEAN && !short_k;
     // groups of gm m-tiles that never mix experts (the 256-row paths, when the mean expert fills a
     // group: C2 -1 %; with Zipf loads, whose remainders then collect at the end of the list from
     // many experts, C5 dlhs ran 1-3 % slower): see build_tiles_kernel
@@ -2709,8 +2717,8 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
     if (mode != 2 && Nout % 256 == 0) {
       const int64_t nks = Kred / mf::v3::BKS;
       const int ncu4 = cus_per_xcd();
-      if (big_m && !gath && nks >= 4 && nks <= MTX_V4P_MAX_STAGES && ncu4 >= 1) {
-        // short reductions: persistent workgroups, the ring running across tiles
+      if (big_m && !gath && nks >= 4 && short_k && (M / E) >= MTX_V4P_MIN_MEAN && ncu4 >= 1) {
+        // short reductions over large groups: persistent workgroups, the ring running across tiles
         rc = launch_build_tiles(gs, E, M, 256, wsp, st, false, false, spread, align);
         if (rc) return rc;
         const int64_t tiles = gmm_max_tiles(M, E, 256) * (Nout / 256);
