@@ -114,8 +114,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const T* __restrict__ x
 }
 
 // One workgroup per 128x128 (Kin x Kout) block of one expert: one scale for the block, codes
-// written transposed ([E, Kout, Kin], k contiguous) through LDS.
-template <typename T, bool P2 = false>
+// written transposed ([E, Kout, Kin], k contiguous) through LDS.  HBM-bound; NT: weights and codes past
+// the caches (64 x [2048, 2816] bf16: 210 us cached, 200 streamed, 208 with only the loads and 210 with
+// only the stores streamed; 64 x [1408, 2048]: 108, 94, 88, 100).
+template <typename T, bool P2, bool NT>
 __global__ __launch_bounds__(256) void quant_weights_kernel(const T* __restrict__ w, int64_t Kin, int64_t Kout,
                                                             uint8_t* __restrict__ wq, float* __restrict__ ws) {
   __shared__ __attribute__((aligned(16))) uint8_t tt[128 * q8::TSTRIDE];
@@ -123,7 +125,7 @@ __global__ __launch_bounds__(256) void quant_weights_kernel(const T* __restrict_
   using S = q8::TileShape<T>;
   const int64_t e = blockIdx.z, k0 = (int64_t)blockIdx.y * 128, n0 = (int64_t)blockIdx.x * 128;
   q8::Tile<T> t;
-  t.load(w + (e * Kin + k0) * Kout + n0, Kout, 128);
+  t.template load<NT>(w + (e * Kin + k0) * Kout + n0, Kout, 128);
   float m[S::VE];
   t.col_amax(m);
   float a = 0.0f;
@@ -132,7 +134,7 @@ __global__ __launch_bounds__(256) void quant_weights_kernel(const T* __restrict_
   const float s = q8::block_scale<P2>(a, red);
   q8::codes_to_lds_t(t, [&](int) { return s; }, tt);
   __syncthreads();
-  q8::lds_t_to_global(tt, wq + (e * Kout + n0) * Kin + k0, Kin);
+  q8::lds_t_to_global<NT>(tt, wq + (e * Kout + n0) * Kin + k0, Kin);
   if (threadIdx.x == 0) ws[(e * (Kout / 128) + blockIdx.x) * (Kin / 128) + blockIdx.y] = s;
 }
 
@@ -1355,12 +1357,20 @@ static int quant_weights_entry(const void* w, int dtype, int64_t E, int64_t Kin,
   if (E > 65535 || Kin / 128 > 65535) return MTX_ERR_UNSUPPORTED;
   dim3 grid((unsigned)(Kout / 128), (unsigned)(Kin / 128), (unsigned)E);
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == MTX_F32)
-    hipLaunchKernelGGL((f8::quant_weights_kernel<float, P2>), grid, dim3(256), 0, st, (const float*)w, Kin, Kout,
-                       w_q, w_scale);
-  else
-    hipLaunchKernelGGL((f8::quant_weights_kernel<uint16_t, P2>), grid, dim3(256), 0, st, (const uint16_t*)w, Kin,
-                       Kout, w_q, w_scale);
+  // streamed once weights and codes pass half of the 256 MB cache (88 x [384, 768], 78 MB: 15.5 us
+  // cached, 16.3 streamed)
+  const bool nt = E * Kin * Kout * (dtype == MTX_F32 ? 5 : 3) >= (int64_t)128 << 20;
+#define MTX_LAUNCH(T, NT)                                                                                      \
+  hipLaunchKernelGGL((f8::quant_weights_kernel<T, P2, NT>), grid, dim3(256), 0, st, (const T*)w, Kin, Kout, w_q, \
+                     w_scale)
+  if (dtype == MTX_F32) {
+    if (nt) MTX_LAUNCH(float, true);
+    else MTX_LAUNCH(float, false);
+  } else {
+    if (nt) MTX_LAUNCH(uint16_t, true);
+    else MTX_LAUNCH(uint16_t, false);
+  }
+#undef MTX_LAUNCH
   return check_launch();
 }
 

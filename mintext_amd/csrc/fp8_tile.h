@@ -34,6 +34,8 @@ struct Tile {
   u32x4 raw[S::G4][4];
   int cl, rl;
 
+  // NT: data read once by one workgroup (weights), loaded past the caches
+  template <bool NT = false>
   __device__ __forceinline__ void load(const T* __restrict__ src, int64_t ld, int nrows) {
     const int tid = threadIdx.x;
     cl = tid % S::LPR;
@@ -44,7 +46,10 @@ struct Tile {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int r = 4 * (rl + S::TR * h) + q;
-        raw[h][q] = r < nrows ? *(const u32x4*)(p + (int64_t)r * ld) : u32x4{0u, 0u, 0u, 0u};
+        if constexpr (NT)
+          raw[h][q] = r < nrows ? __builtin_nontemporal_load((const u32x4*)(p + (int64_t)r * ld)) : u32x4{0u, 0u, 0u, 0u};
+        else
+          raw[h][q] = r < nrows ? *(const u32x4*)(p + (int64_t)r * ld) : u32x4{0u, 0u, 0u, 0u};
       }
   }
   // element j (column cl*VE + j) of load (h, q) as float
@@ -117,6 +122,7 @@ __device__ __forceinline__ void codes_to_lds_t(const Tile<T>& t, SC sc, uint8_t*
 }
 
 // 128 transposed rows of 128 bytes from LDS to dst + c * ld (16 bytes per lane, 8 lanes per row)
+template <bool NT = false>
 __device__ __forceinline__ void lds_t_to_global(const uint8_t* tt, uint8_t* __restrict__ dst, int64_t ld) {
   const int tid = threadIdx.x, seg = tid & 7;
 #pragma unroll
@@ -125,7 +131,8 @@ __device__ __forceinline__ void lds_t_to_global(const uint8_t* tt, uint8_t* __re
     const uint8_t* s = tt + c * TSTRIDE + seg * 16;
     const u32x4 v{*(const uint32_t*)s, *(const uint32_t*)(s + 4), *(const uint32_t*)(s + 8),
                   *(const uint32_t*)(s + 12)};
-    *(u32x4*)(dst + (int64_t)c * ld + seg * 16) = v;
+    if constexpr (NT) __builtin_nontemporal_store(v, (u32x4*)(dst + (int64_t)c * ld + seg * 16));
+    else *(u32x4*)(dst + (int64_t)c * ld + seg * 16) = v;
   }
 }
 
