@@ -26,13 +26,16 @@ _ROWS, _GATHER, _SWIGLU = 0, 1, 2
 
 
 def experts_fp8_train_supported(x, topk_indices, topk_weights, gate_up, down, scales) -> bool:
-    """Whether ``experts_fp8_train`` takes these arguments: bf16 tokens, widths in tiles of 256 and
-    32-bit operand offsets (the other forms, and what has to raise, take the separate steps)."""
+    """Whether ``experts_fp8_train`` takes these arguments: bf16 tokens, widths in tiles of 256,
+    tokens aligned for 16-byte loads (a sorted copy of others is) and 32-bit operand offsets (the other
+    forms, and what has to raise, take the separate steps)."""
     if scales not in SCALE_MODES or x.dtype != torch.bfloat16 or x.dim() != 2 or topk_indices.dim() != 2:
         return False
     if gate_up.dim() != 3 or down.dim() != 3 or gate_up.dtype != down.dtype:
         return False
     if gate_up.dtype not in (torch.bfloat16, torch.float32) or topk_weights.dtype not in (torch.bfloat16, torch.float32):
+        return False
+    if x.is_contiguous() and x.data_ptr() % 16:
         return False
     N, D = x.shape
     E, D2, two_i = gate_up.shape

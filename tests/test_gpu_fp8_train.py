@@ -85,3 +85,17 @@ def test_no_gradient_and_changed_weights(dev):
         gu.mul_(2.0)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         out.backward(dout)
+
+
+@pytest.mark.parametrize("offset", [1, 4, 8])
+def test_tokens_at_any_offset(dev, offset):
+    """Tokens that start off a 16-byte boundary take the separate steps, whose sorted copy is aligned."""
+    from mintext_amd.kernels.fp8_train import experts_fp8_train_supported
+    from mintext_amd.moe import moe_experts_forward_fp8_train
+
+    x, idx, w, gu, dn, _ = _inputs(dev, 65, 256, 4, 2, 256, torch.bfloat16)
+    moved = torch.empty(x.numel() + offset, dtype=x.dtype, device=dev)[offset:].view(x.shape)
+    moved.copy_(x)
+    assert experts_fp8_train_supported(moved, idx, w, gu, dn, "amax") == (offset == 8)
+    got = moe_experts_forward_fp8_train(moved, idx, w, gu, dn, scales="amax")
+    assert torch.equal(got, moe_experts_forward_fp8_train(x, idx, w, gu, dn, scales="amax"))
