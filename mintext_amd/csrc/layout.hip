@@ -7,8 +7,8 @@
 // (column offset = pointer offset, row stride 2I), or reads them back.  Element size 2 or 4
 // bytes.  HBM-bound: 2 * B * R * C * elem bytes per call.
 //
-// Whole wave tiles (64x64 bf16, 32x32 f32; 16-byte aligned) turn in registers; sizes with a remainder
-// take transpose_batched_kernel.  There a workgroup moves one 64x64 tile: 16-byte coalesced loads of 64 input rows into LDS, then
+// Whole wave tiles (64x64 bf16, 32x32 f32; 16-byte aligned) of large calls turn in registers; the rest
+// takes transpose_batched_kernel.  There a workgroup moves one 64x64 tile: 16-byte coalesced loads of 64 input rows into LDS, then
 // 16-byte coalesced stores of 64 output rows read down the LDS columns (rows padded by one
 // 16-byte chunk so that the column reads spread over the banks).  Tiles that are ragged or not
 // 16-byte aligned take a per-element path.
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void transpose_batched_kernel(const T* __restr
 // of lanes, each with an 8 x 8 (4 x 4) block.  Eight lanes load a 128-byte line of an input row and
 // eight store one of an output row; the block turns in registers (byte permutes), so there is no LDS,
 // no barrier, and all of a wave's loads are in flight at once.  Waves are numbered along the input's
-// rows (512 contiguous bytes per workgroup) with none idle at a row's end.  NT: both sides bypass the
+// rows (512 contiguous bytes per workgroup) with none idle at a row's end.  Both sides bypass the
 // caches, which data read and written once would only sweep.
 // 64 x [1408, 2048] bf16 into rows of 2816: LDS tiles 148 us, this with 2 x 2 waves 138 (cached loads 140,
 // cached stores 145), with four along a row 131 (5.6 TB/s; a plain copy reaches 5.9-6.1), down a column 150.
@@ -92,7 +92,7 @@ __device__ __forceinline__ void transpose_block(const u32x4 (&in)[4], u32x4 (&ou
 #pragma unroll
     for (int q = 0; q < 4; ++q) out[j][q] = in[q][j];
 }
-template <typename T, bool NT>
+template <typename T>
 __global__ __launch_bounds__(256) void transpose_tiles_kernel(const T* __restrict__ in, int64_t in_bs, int64_t in_ld,
                                                               T* __restrict__ out, int64_t out_bs, int64_t out_ld,
                                                               int tiles_r, int tiles_c) {
@@ -104,17 +104,11 @@ __global__ __launch_bounds__(256) void transpose_tiles_kernel(const T* __restric
   u32x4 v[B], w[B];
   const T* src = in + blockIdx.z * in_bs + (r + (lane >> 3) * B) * in_ld + c + (lane & 7) * B;
 #pragma unroll
-  for (int i = 0; i < B; ++i) {
-    if constexpr (NT) v[i] = __builtin_nontemporal_load((const u32x4*)(src + i * in_ld));
-    else v[i] = *(const u32x4*)(src + i * in_ld);
-  }
+  for (int i = 0; i < B; ++i) v[i] = __builtin_nontemporal_load((const u32x4*)(src + i * in_ld));
   transpose_block(v, w);
   T* dst = out + blockIdx.z * out_bs + (c + (lane & 7) * B) * out_ld + r + (lane >> 3) * B;
 #pragma unroll
-  for (int j = 0; j < B; ++j) {
-    if constexpr (NT) __builtin_nontemporal_store(w[j], (u32x4*)(dst + j * out_ld));
-    else *(u32x4*)(dst + j * out_ld) = w[j];
-  }
+  for (int j = 0; j < B; ++j) __builtin_nontemporal_store(w[j], (u32x4*)(dst + j * out_ld));
 }
 
 }  // namespace lay
@@ -137,23 +131,21 @@ extern "C" int mtx_transpose_batched(const void* in, int dtype, int64_t B, int64
   const int64_t tiles_c = ceil_div(C, lay::TILE);
   if (tiles_c > INT32_MAX) return MTX_ERR_ARG;
   hipStream_t st = (hipStream_t)stream;
+  // Whole tiles of 128 MB (half the memory-side cache) or more: streamed through registers.  Below that
+  // the next reader finds the data in the cache, and the LDS tiles are ahead at most sizes.  A whole
+  // import with its fp8 codes, bf16, E x D x I, us with LDS / register tiles: 36 x 768 x 768 (85 MB a
+  // transpose) 88.8 / 95.9, 64 x 768 x 640 (126 MB) 121 / 130, 88 x 384 x 512 (69 MB) 75.5 / 79.0, but
+  // 64 x 512 x 512 (67 MB) 72.5 / 69.9 and 8 x 1024 x 1024 (34 MB) 47.9 / 42.3; above the line
+  // 64 x 1024 x 768 (201 MB) 221 / 196, 64 x 2048 x 1408 (738 MB) 744 / 685.
   const int64_t wt = 8 * epc, wtiles = ceil_div(R, wt) * ceil_div(C, wt);  // wave tiles
-  if (vec_ok && R % wt == 0 && C % wt == 0 && wtiles <= INT32_MAX - 3) {
-    // past half of the 256 MB cache the data leaves it before a next reader comes: streamed
-    // (88 x [384, 512] bf16, 69 MB: 12.8 us cached, 14.5 streamed; 369 MB: 140 cached, 138 streamed)
-    const bool nt = 2 * B * R * C * es >= (int64_t)128 << 20;
-    dim3 grid((unsigned)ceil_div(wtiles, 4), 1, (unsigned)B);
-#define MTX_LAUNCH(T, NT)                                                                                        \
-  hipLaunchKernelGGL((lay::transpose_tiles_kernel<T, NT>), grid, dim3(256), 0, st, (const T*)in, in_batch_stride, \
-                     in_ld, (T*)out, out_batch_stride, out_ld, (int)(R / wt), (int)(C / wt))
-    if (dtype == MTX_F32) {
-      if (nt) MTX_LAUNCH(float, true);
-      else MTX_LAUNCH(float, false);
-    } else {
-      if (nt) MTX_LAUNCH(uint16_t, true);
-      else MTX_LAUNCH(uint16_t, false);
-    }
-#undef MTX_LAUNCH
+  if (vec_ok && R % wt == 0 && C % wt == 0 && wtiles <= INT32_MAX - 3 && 2 * B * R * C * es >= (int64_t)128 << 20) {
+    dim3 tiles((unsigned)ceil_div(wtiles, 4), 1, (unsigned)B);
+    if (dtype == MTX_F32)
+      hipLaunchKernelGGL(lay::transpose_tiles_kernel<float>, tiles, dim3(256), 0, st, (const float*)in, in_batch_stride,
+                         in_ld, (float*)out, out_batch_stride, out_ld, (int)(R / wt), (int)(C / wt));
+    else
+      hipLaunchKernelGGL(lay::transpose_tiles_kernel<uint16_t>, tiles, dim3(256), 0, st, (const uint16_t*)in,
+                         in_batch_stride, in_ld, (uint16_t*)out, out_batch_stride, out_ld, (int)(R / wt), (int)(C / wt));
     return check_launch();
   }
   dim3 grid((unsigned)tiles_c, (unsigned)ceil_div(R, lay::TILE), (unsigned)B);

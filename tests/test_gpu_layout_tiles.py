@@ -22,6 +22,7 @@ def _transpose(x, out, R, C, out_bs, out_ld, offset=0):
     (1, 32, 32), (1, 64, 64), (3, 64, 192), (2, 320, 64), (2, 192, 320), (2, 96, 160), (2, 72, 64), (2, 64, 72),
     (16, 1024, 2048), (33, 1024, 1024),  # 67 and 69 MB in and out for bf16, 134 and 138 MB for f32
     (64, 1024, 1024),  # 268 MB in and out for bf16: streamed
+    (5500, 64, 192), (2800, 96, 160),  # streamed, 3 (bf16) and 15 (f32) wave tiles: the last workgroup partly empty
 ])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 def test_transpose_tiles(dev, B, R, C, dt):
