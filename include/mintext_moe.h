@@ -190,7 +190,7 @@ int mtx_unroute_bwd(const void* dout, int g_dtype, const void* sorted_output, in
 
 /* ---- grouped GEMM ----------------------------------------------------------------------
  * Rows of x are grouped contiguously in group_sizes order (a device array that is never
- * read on the host).  Rows past sum(group_sizes) produce zeros.  F32 (exact fp32 FMA) or
+ * read on the host).  Rows past sum(group_sizes) produce zeros.  F32 (f32 MFMA: f32 products and sums) or
  * BF16 (MFMA, f32 accumulate, one rounding).  Output dtype = input dtype.
  * The workspace holds the per-call tile lists and (64 MB) the f32 partial tiles of the
  * split tail: on the 256-row bf16 path, when an XCD's last round of output tiles is at most
