@@ -1464,6 +1464,9 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
   {
     const int frow = lane & 31, h4 = 4 * (lane >> 5);
     if constexpr (EPI == EPI_SWIGLU) {
+      // EDGE widths keep the accurate function: swiglu_fast's product g * u may overflow where the result
+      // does not, and gives NaN once exp(-g) does
+      auto act = [](float g, float u) { return EDGE ? silu_f32(g) * u : swiglu_fast(g, u); };
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -1473,8 +1476,8 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
             const f32x16& gt = acc[i][j];
             const f32x16& up = acc[i][j + TN / 2];
             stage8(wm * WTM + i * 32 + frow, wn * (WTN / 2) + j * 32 + 8 * g + h4,
-                   pack4(swiglu_fast(gt[4 * g], up[4 * g]), swiglu_fast(gt[4 * g + 1], up[4 * g + 1]),
-                         swiglu_fast(gt[4 * g + 2], up[4 * g + 2]), swiglu_fast(gt[4 * g + 3], up[4 * g + 3])));
+                   pack4(act(gt[4 * g], up[4 * g]), act(gt[4 * g + 1], up[4 * g + 1]),
+                         act(gt[4 * g + 2], up[4 * g + 2]), act(gt[4 * g + 3], up[4 * g + 3])));
           }
     } else {
 #pragma unroll
@@ -2648,6 +2651,10 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
     t.Kred = (int)Kred;
     t.N = (int)Nout;
     t.I = (int)(mode == 2 ? I : 0);
+    // a layer's SwiGLU does not depend on its number of rows: the function of the kernel that larger
+    // groups of these widths run on
+    t.fast_silu = I % 128 == 0 && Kred % mf::BK == 0 && (gath ? gather_rows : M) * Kred * 2 < (int64_t(1) << 32) &&
+                  Kred * Nout * 2 < (int64_t(1) << 32);
     return launch_gmm_thin(t, st);
   }
   auto base_args = [&]() {

@@ -15,6 +15,7 @@ struct ThinArgs {
   int gather_div, gather_rows;
   int M, E, Kred, N;
   int I;                 // SwiGLU: N = 2 I, gate columns first; 0: plain store
+  int fast_silu;         // SwiGLU with the hardware exp2 and reciprocal; 0: silu_f32
 };
 
 // Whether launch_gmm_thin takes (and is the faster kernel for) M rows in E groups of Kred x N: widths

@@ -179,7 +179,7 @@ __global__ __launch_bounds__(NW * 64) void gmm_thin_kernel(ThinArgs p) {
       if (SWIGLU) {
         const f32x4 u = FORM == WIDE ? sum4(KW, tok, c) : sum4(0, tok, 64 + c);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = swiglu_fast(v[q], u[q]);
+        for (int q = 0; q < 4; ++q) v[q] = p.fast_silu ? swiglu_fast(v[q], u[q]) : silu_f32(v[q]) * u[q];
       }
       *(bf16x4*)(p.C + (int64_t)row * ocols + oc) = bf16x4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
     }
