@@ -22,8 +22,9 @@
 // of tgmm) keep their natural layout and are turned into MFMA operands by ds_read_b64_tr_b16
 // (gfx950 transpose read).  The epilogue (SwiGLU fused for gate_up) stages the tile through the
 // idle ring and writes whole 128-byte lines.  gmm_mfma_kernel, an earlier register-staged design
-// (two LDS buffers, 8x8 register transposes), runs only the shapes whose operands exceed 32-bit
-// byte offsets.
+// (two LDS buffers, 8x8 register transposes), runs widths that are odd multiples of 128 where the
+// 256-row tiles would be few or mostly padding, and what the ring kernels do not take: operands beyond
+// 32-bit byte offsets and, at those widths, outputs off a 16-byte boundary.
 // f32 path (and bf16 widths that are no multiple of 8): f32 MFMA tiles staged through LDS.
 #include "common.h"
 #include "gmm_thin.h"
@@ -2761,9 +2762,16 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
       return mode == 0 ? launch_mfma<128, 256, 1, 2, mf::FWD, mf::EPI_STORE>(a, grid, st)
                        : launch_mfma<128, 256, 1, 2, mf::DLHS, mf::EPI_STORE>(a, grid, st);
     }
-    // Nout a multiple of 128 but not of 256: the ring kernel's EDGE form below is faster (8192 rows
-    // in 8 groups, 1024 x 1408: 55 -> 37 us, its dlhs 49 -> 38 us); this one keeps what that cannot take
-    if (mode != 2 && Nout % 128 == 0 && (!v3ok || (uintptr_t)out % 16 != 0)) {
+    // Nout a multiple of 128 but not of 256: 128x128 tiles, unless the 256-row ring kernel's EDGE form
+    // (below) can take the call and is ahead.  It needs two rounds of its four times larger tiles on 256
+    // CUs, groups that fill them and little padding (us, 128x128 / EDGE, forward): 16384 rows in 8
+    // groups, 2048 x 1408 153 / 127; 32 groups, 2048 x 1920 248 / 191.  Short of that 4096 rows in 8 groups,
+    // 2048 x 1408 (144 tiles) 55 / 59, its dlhs 46 / 57; 2048 x 128 (half of each tile is padding) 41 / 54,
+    // dlhs 32 / 52; Zipf loads of 4096 rows in 128 groups, 1024 x 896 (many small groups) 61 / 73, dlhs
+    // 53 / 70.
+    const int64_t edge_tiles = (M / 256 + E) * ceil_div(Nout, 256);
+    const bool edge_ahead = M / E >= 256 && edge_tiles >= 512 && Nout >= 640;
+    if (mode != 2 && Nout % 128 == 0 && (!v3ok || (uintptr_t)out % 16 != 0 || !edge_ahead)) {
       rc = launch_build_tiles(gs, E, M, 128, wsp, st);
       if (rc) return rc;
       const int64_t grid = gmm_max_tiles(M, E, 128) * (Nout / 128);
@@ -2997,8 +3005,13 @@ extern "C" int mtx_tgmm(const void* x, const void* g, const int32_t* group_sizes
       const int64_t grid = round_up(E * (K / 256) * (N / 256), 8);
       return launch_mfma<256, 256, 2, 2, mf::TGMM, mf::EPI_STORE>(a, grid, st);
     }
-    // (8192 rows in 8 groups, 1408 x 1024: 58 us here, 38 us in the ring kernel's EDGE form below)
-    if ((uintptr_t)dw % 16 != 0 || M * K * 2 >= (int64_t(1) << 32) || M * N * 2 >= (int64_t(1) << 32)) {
+    // 128x128 tiles, or the ring kernel's EDGE form below where its 256x256 tiles keep half of the chip
+    // busy and are at most a third padding (us, 128x128 / EDGE): 16384 rows in 8 groups, 1408 x 1024 101 / 65,
+    // 4096 rows in 32 groups, 384 x 1024 25 / 21; but 4096 rows in 8 groups, 384 x 1024 (64 tiles) 22 / 24, 16384
+    // rows in 8 groups, 640 x 640 (72 tiles) 51 / 56, in 32 groups, 128 x 1024 (half padding) 24 / 26.
+    const int64_t tk = ceil_div(K, 256), tn = ceil_div(N, 256);
+    const bool edge_ahead = E * tk * tn >= 128 && 2 * tk * tn * 65536 <= 3 * K * N;
+    if ((uintptr_t)dw % 16 != 0 || M * K * 2 >= (int64_t(1) << 32) || M * N * 2 >= (int64_t(1) << 32) || !edge_ahead) {
       const int64_t grid = round_up(E * (K / 128) * (N / 128), 8);
       return launch_mfma<128, 128, 2, 2, mf::TGMM, mf::EPI_STORE>(a, grid, st);
     }

@@ -51,3 +51,15 @@ def tile_list_workspace_bytes(M: int, E: int) -> int:
     tail): with it every tile runs whole, so any two kernels agree bit for bit."""
     up = lambda a, b: (a + b - 1) // b * b
     return up(up((48 + 2 * E + 1) * 4, 256) + (-(-M // 64) + E + 1) * 16, 256)
+
+
+def launched(f) -> str:
+    """The names of the kernels that ``f`` launches, one a line."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as p:
+        f()
+        torch.cuda.synchronize()
+    return "\n".join(e.name for e in p.events() if e.device_type == torch.autograd.DeviceType.CUDA)
