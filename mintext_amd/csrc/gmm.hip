@@ -57,15 +57,27 @@ struct GmmWs {
 // Split tail (256x256 store tiles, FWD/DLHS).  Workgroup pid is dispatched to XCD pid % 8 and
 // each CU holds one 256-row workgroup, so an XCD runs its tiles in rounds of (CUs per XCD).
 // When the last round holds at most half as many tiles as CUs (rem <= kSplitMaxRem), those rem
-// tiles are split along K into S = min(kSplitMaxS, CUs / rem) pieces, dispatched after the
+// tiles are split along K into up to min(kSplitMaxS, CUs / rem) pieces, dispatched after the
 // whole tiles; each piece stores an f32 partial tile, and the piece that arrives last (per-tile
 // counter) sums the partials in piece order and runs the epilogue.  No workgroup waits on
 // another, and the sum does not depend on arrival order.  The dispatch assumption only
 // affects speed: any placement gives the same result.  At most kSplitItems pieces per XCD.
 // A piece holds at least kSplitMinStages 32-k stages: exchanging the partials costs 8-15 us, so a
 // shorter reduction loses (8192 rows in 8 groups x Kred x 2048, split / whole: Kred 1408 84 / 68 us,
-// 2048 100 / 92, 4096 159 / 165, 14336 489 / 527; 2000 rows x 7168 x 1024: 80 / 175).
+// 2048 100 / 92, 4096 159 / 165, 14336 489 / 527; 2000 rows x 7168 x 1024: 80 / 175).  Where an XCD has at
+// most kSplitFewTiles tiles in all, the call is one tile's reduction on an idle chip and few pieces share
+// the exchange: there kSplitMinStages or more are split into pieces of at least kSplitFewStagesV3 (256 rows
+// in one group, 2048 x 512, whole / pieces of 24 stages / of 16: 46 / 37 / 33 us; means of such calls against
+// whole tiles: 40 stages 0.97, 48 0.86, 64 0.75, but 32 1.03).  The one-wave-per-SIMD kernel's pieces cost
+// twice as much to exchange (its 64 stages in two pieces 0.93, 48 1.04).
 constexpr int kSplitXcd = 8, kSplitItems = 32, kSplitMaxRem = 16, kSplitMaxS = 4, kSplitMinStages = 40;
+constexpr int kSplitFewTiles = 8, kSplitFewStagesV3 = 16, kSplitFewStagesW4 = 32;
+// Pieces of each tile of the last round: `tiles` of the XCD, `rem` of them in that round.
+__device__ __forceinline__ int split_pieces(int tiles, int rem, int ncu, int stages, int few_stages) {
+  if (rem <= 0 || rem > kSplitMaxRem || 2 * rem > ncu || stages < kSplitMinStages) return 1;
+  const int per = tiles <= kSplitFewTiles ? few_stages : kSplitMinStages;
+  return min(min(kSplitMaxS, ncu / rem), max(stages / per, 1));
+}
 constexpr int64_t kSplitSlotFloats = 256 * 256;
 static inline int64_t gmm_ws_tiles_off(int64_t E) { return round_up((int64_t)(48 + 2 * E + 1) * 4, 256); }
 static inline int64_t gmm_max_tiles(int64_t M, int64_t E, int64_t BM) { return ceil_div(M, BM) + E + 1; }
@@ -1139,8 +1151,7 @@ __global__ __launch_bounds__(WM* WN * 64, MTX_V3_WPE) void gmm_v3_kernel(Args p)
       // pieces, dispatched after the whole tiles
       const int tx = max(0, min(per, total - xcd * per));
       const int rem = tx % p.ncu_x;
-      int S = (rem > 0 && rem <= kSplitMaxRem && 2 * rem <= p.ncu_x) ? min(kSplitMaxS, p.ncu_x / rem) : 1;
-      S = min(S, max(p.Kred / BKS / kSplitMinStages, 1));
+      const int S = split_pieces(tx, rem, p.ncu_x, p.Kred / BKS, kSplitFewStagesV3);
       const int nwhole = (S > 1) ? tx - rem : tx;
       if (q >= nwhole + (S > 1 ? rem * S : 0)) return;
       if (q < nwhole) {
@@ -2350,8 +2361,7 @@ __global__ __launch_bounds__(256, 1) void gmm_w4_kernel(Args p) {
     S = 1;
     if (EPI == EPI_STORE && p.split_on) {
       const int rem = tx % p.ncu_x;
-      int S_ = (rem > 0 && rem <= kSplitMaxRem && 2 * rem <= p.ncu_x) ? min(kSplitMaxS, p.ncu_x / rem) : 1;
-      S_ = min(S_, max(p.Kred / v3::BKS / kSplitMinStages, 1));
+      const int S_ = split_pieces(tx, rem, p.ncu_x, p.Kred / v3::BKS, kSplitFewStagesW4);
       if (S_ > 1) {
         nwhole = tx - rem;
         S = S_;

@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("op", ["fwd", "dlhs"])
 @pytest.mark.parametrize("M,E,Kred,N", [
-    (300, 2, 1280, 1024),    # 40 stages: too short for two pieces
+    (300, 2, 1248, 1024),    # 39 stages: too short for two pieces
+    (300, 2, 1280, 1024),    # few tiles: 40 stages in two pieces
     (300, 2, 2560, 1024),    # two pieces, the wave rows of some of them empty
     (1100, 2, 2592, 2048),   # pieces of unequal length
     (700, 3, 5120, 512),     # four pieces
@@ -46,5 +47,7 @@ def test_split_tail_equals_whole_tiles(dev, op, M, E, Kred, N):
     whole = call(tile_list_workspace_bytes(M, E))
     split = call(full)
     again = call(full)
+    # some of the f32 sums round to another bf16 value when they are added in pieces
+    assert torch.equal(split, whole) == (Kred < 1280)
     assert torch.equal(split, again)  # summed in piece order, whatever the order of arrival
     assert ((split - whole).abs() <= whole.abs() * 2.0 ** -7 + whole.abs().max() * 2.0 ** -16).all()
