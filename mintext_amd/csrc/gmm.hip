@@ -347,34 +347,48 @@ constexpr int CS = 64 + 8;  // LDS row of an operand stored [k][64]: the half-wa
 constexpr int TILE = 64 * RS > KS * CS ? 64 * RS : KS * CS;
 
 // One operand tile of 64 rows x KS reduction elements (COLS = false: the reduction contiguous in
-// memory) or KS reduction elements x 64 columns (COLS = true).  at(r, c, v) says whether row r,
-// column c exists and where it is.
+// memory) or KS reduction elements x 64 columns (COLS = true).  at(r, c) is where row r, column c is,
+// or nullptr.
 template <typename T, bool COLS, int VEC>
 struct Stage {
   static_assert(VEC == 1 || std::is_same<T, float>::value, "16-byte loads are of f32");
   static constexpr int W = COLS ? 64 : KS, H = COLS ? KS : 64, N = W * H / NT / VEC;
-  float v[N][VEC];
+  // bf16: values as loaded and a bit for each that exists; the others load `any`, a valid address.  A load
+  // with its conversion inside the condition was waited for before the next one was issued (tgmm of 4096
+  // rows in 4 groups, 500 x 250: 167 us, 81 this way; f32 needs no conversion and is faster with the
+  // condition).  Reduction elements past `left` (a multiple of 8) are skipped.
+  static constexpr bool BF16 = std::is_same<T, uint16_t>::value;
+  T v[N][VEC];
+  uint32_t have;
+  static_assert(!BF16 || N <= 32, "a bit a value");
   template <typename At>
-  __device__ __forceinline__ void load(At at, int tid) {
+  __device__ __forceinline__ void load(At at, const T* any, int left, int tid) {
+    have = 0;
 #pragma unroll
     for (int u = 0; u < N; ++u) {
       const int q = tid + u * NT, r = q / (W / VEC), c = q % (W / VEC) * VEC;
+      if (BF16 && COLS && r >= left) continue;
       const T* src = at(r, c);
-      if constexpr (VEC == 4) {
+      if constexpr (BF16) {
+        v[u][0] = *(src ? src : any);
+        have |= src ? 1u << u : 0u;
+      } else if constexpr (VEC == 4) {
         const f32x4 x = src ? *(const f32x4*)src : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[u][i] = x[i];
       } else {
-        v[u][0] = src ? gld<T>(src, 0) : 0.0f;
+        v[u][0] = src ? *src : 0.0f;
       }
     }
   }
-  __device__ __forceinline__ void store(float* lds, int tid) const {
+  __device__ __forceinline__ void store(float* lds, int left, int tid) const {
 #pragma unroll
     for (int u = 0; u < N; ++u) {
       const int q = tid + u * NT, r = q / (W / VEC), c = q % (W / VEC) * VEC;
+      if (BF16 && COLS && r >= left) continue;
       float* dst = lds + r * (COLS ? CS : RS) + c;
       if constexpr (VEC == 4) *(f32x4*)dst = f32x4{v[u][0], v[u][1], v[u][2], v[u][3]};
+      else if constexpr (BF16) *dst = (have >> u) & 1 ? bf16_to_f32(v[u][0]) : 0.0f;
       else *dst = v[u][0];
     }
   }
@@ -397,29 +411,40 @@ __device__ __forceinline__ void fragment(const float* lds, int x0, int lane, flo
   }
 }
 // acc of lane l, element v: row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32 of the wave's 32x32 tile.
+// nred: reduction elements; any_a, any_b: valid addresses of the operands (for nred > 0).
 template <typename T, bool ACOLS, bool BCOLS, int VEC, typename AtA, typename AtB>
-__device__ __forceinline__ void mainloop(f32x16& acc, int nk, float* as, float* bs, AtA at_a, AtB at_b) {
+__device__ __forceinline__ void mainloop(f32x16& acc, int nred, float* as, float* bs, AtA at_a, AtB at_b, const T* any_a,
+                                         const T* any_b) {
+  constexpr bool BF16 = std::is_same<T, uint16_t>::value;
+  const int nk = (nred + KS - 1) / KS;
   const int tid = threadIdx.x, lane = tid & 63, wm = (tid >> 6) >> 1, wn = (tid >> 6) & 1;
   Stage<T, ACOLS, VEC> a;
   Stage<T, BCOLS, VEC> b;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+  // bf16: a last stage of few elements (tgmm of small groups) does no more than the eights of them
+  auto elements = [&](int s) { return BF16 ? min(KS, (nred - s * KS + 7) & ~7) : KS; };
   auto load = [&](int s) {
-    a.load([&](int r, int c) { return at_a(r, c, s); }, tid);
-    b.load([&](int r, int c) { return at_b(r, c, s); }, tid);
+    a.load([&](int r, int c) { return at_a(r, c, s); }, any_a, elements(s), tid);
+    b.load([&](int r, int c) { return at_b(r, c, s); }, any_b, elements(s), tid);
   };
   if (nk > 0) load(0);
   // one LDS buffer: a second one saves a barrier a stage but halves the workgroups per CU (5-9 % slower)
   for (int s = 0; s < nk; ++s) {
-    a.store(as, tid);
-    b.store(bs, tid);
+    const int left = elements(s);
+    a.store(as, left, tid);
+    b.store(bs, left, tid);
     __syncthreads();
     if (s + 1 < nk) load(s + 1);
     float fa[16], fb[16];
     fragment<ACOLS>(as, wm * 32, lane, fa);
     fragment<BCOLS>(bs, wn * 32, lane, fb);
 #pragma unroll
-    for (int m = 0; m < 16; ++m) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[m], fb[m], acc, 0, 0, 0);
+    for (int q = 0; q < 4; ++q) {
+      if (BF16 && 8 * q >= left) continue;
+#pragma unroll
+      for (int m = 4 * q; m < 4 * q + 4; ++m) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[m], fb[m], acc, 0, 0, 0);
+    }
     __syncthreads();
   }
 }
@@ -465,7 +490,7 @@ __global__ __launch_bounds__(NT) void gmm_kernel(const T* __restrict__ A, const 
     return n < Nout && k < Kred ? We + k * Nout + n : nullptr;
   };
   f32x16 acc;
-  mainloop<T, false, MODE != 1, VEC>(acc, (int)((Kred + KS - 1) / KS), as, bs, at_a, at_b);
+  mainloop<T, false, MODE != 1, VEC>(acc, (int)Kred, as, bs, at_a, at_b, A + (int64_t)t.r0 * Kred, We);
   const int rb = wm * 32 + 4 * (lane >> 5), col = lane & 31;
   if constexpr (MODE == 2) {
     // the up half through LDS, rows of 32 (the main loop's last barrier is behind every read)
@@ -509,7 +534,7 @@ __global__ __launch_bounds__(NT) void tgmm_kernel(const T* __restrict__ X, const
     return row < r1 && n < N ? G + row * N + n : nullptr;
   };
   f32x16 acc;
-  mainloop<T, true, true, VEC>(acc, (int)((r1 - r0 + KS - 1) / KS), as, bs, at_a, at_b);
+  mainloop<T, true, true, VEC>(acc, (int)(r1 - r0), as, bs, at_a, at_b, X + r0 * K, G + r0 * N);
   const int lane = threadIdx.x & 63, wm = (threadIdx.x >> 6) >> 1, wn = (threadIdx.x >> 6) & 1;
   T* out = dW + (int64_t)e * K * N;
 #pragma unroll

@@ -64,3 +64,24 @@ def test_odd_multiples_of_128_tgmm(dev, E, K, N, ring):
     names = launched(lambda: tgmm(x, dy, g))
     assert ("gmm_v3_kernel" in names, "gmm_mfma_kernel" in names) == (ring, not ring), names
     assert rel_err(f64(tgmm(x, dy, g)), O.tgmm(f64(x), f64(dy), gs)) < TOL
+
+
+# bf16 rows without the alignment that the bf16 tiles need: the f32 matrix tiles, single values; sums that end
+# around the eights and stages of 32 that they are taken in
+@pytest.mark.parametrize("K,N", [(63, 129), (33, 7), (1, 66)])
+@pytest.mark.parametrize("gs", [[1, 7, 8, 9, 0, 31, 32, 33], [100, 0, 3, 65]])
+def test_bf16_odd_widths(dev, K, N, gs):
+    from mintext_amd.kernels import grouped_matmul, tgmm
+    from mintext_amd.kernels.grouped_matmul import _gmm_dlhs
+
+    gs = np.array(gs, np.int32)
+    n, E = int(gs.sum()), len(gs)
+    x, dy, w = _bf16(dev, n + 5, K), _bf16(dev, n + 5, N), _bf16(dev, E, K, N, std=0.05)
+    x[n:] = dy[n:] = float("nan")
+    g = torch.from_numpy(gs).to(dev)
+    assert "f32mm" in launched(lambda: tgmm(x, dy, g))
+    xr, dr = np.nan_to_num(f64(x)), np.nan_to_num(f64(dy))
+    out, dx, dw = f64(grouped_matmul(x, w, g)), f64(_gmm_dlhs(dy, w, g)), f64(tgmm(x, dy, g))
+    assert rel_err(out[:n], O.gmm(xr, f64(w), gs)[:n]) < TOL and (out[n:] == 0).all()
+    assert rel_err(dx[:n], O.gmm(dr, f64(w).transpose(0, 2, 1), gs)[:n]) < TOL and (dx[n:] == 0).all()
+    assert rel_err(dw, O.tgmm(xr, dr, gs)) < TOL and (dw[gs == 0] == 0).all()
