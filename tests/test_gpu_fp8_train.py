@@ -99,3 +99,47 @@ def test_tokens_at_any_offset(dev, offset):
     assert experts_fp8_train_supported(moved, idx, w, gu, dn, "amax") == (offset == 8)
     got = moe_experts_forward_fp8_train(moved, idx, w, gu, dn, scales="amax")
     assert torch.equal(got, moe_experts_forward_fp8_train(x, idx, w, gu, dn, scales="amax"))
+
+
+# few rows per expert (the codes' padding to 128 rows outweighs them), many, a token per row; every choice of
+# what is kept
+@pytest.mark.parametrize("T,D,E,K,I,wdt", [
+    (96, 512, 16, 2, 256, torch.bfloat16), (4096, 512, 8, 4, 256, torch.bfloat16), (2048, 512, 8, 1, 512, torch.float32),
+    (8192, 256, 2, 1, 256, torch.bfloat16), (1024, 1024, 4, 2, 1024, torch.bfloat16),
+])
+def test_memory_of_fused_step(dev, T, D, E, K, I, wdt):
+    """Between its passes, and at the peak of both, a layer holds no more than the separate steps do."""
+    from mintext_amd.kernels.fp8_train import experts_fp8_train
+
+    *t, dout = _inputs(dev, T, D, E, K, I, wdt)
+    used = {}
+    for f in (_steps, experts_fp8_train, _steps, experts_fp8_train):  # the first two also warm the allocator
+        x, idx, w, gu, dn = (a.clone() for a in t)
+        leaves = [a.requires_grad_(True) for a in (x, w, gu, dn)]
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        base = torch.cuda.memory_allocated()
+        out = f(x, idx, w, gu, dn, "amax")
+        held = torch.cuda.memory_allocated() - base
+        grads = torch.autograd.grad(out, leaves, dout)
+        used[f] = (held, torch.cuda.max_memory_allocated() - base)
+        del out, grads
+    slack = 1 << 16  # the allocator rounds each tensor up to 512 bytes
+    for a, b in zip(used[experts_fp8_train], used[_steps]):
+        assert a <= b + slack, used
+
+
+def test_tokens_changed_before_the_backward(dev):
+    """The gradients are of the tokens that the forward saw, as in the separate steps."""
+    from mintext_amd.kernels.fp8_train import experts_fp8_train
+
+    *t, dout = _inputs(dev, 200, 256, 5, 2, 256, torch.bfloat16)
+    got = []
+    for change in (False, True):
+        x, idx, w, gu, dn = (a.clone() for a in t)
+        gu.requires_grad_(True)
+        out = experts_fp8_train(x, idx, w, gu, dn, "amax")
+        if change:
+            x.zero_()
+        got.append(torch.autograd.grad(out, gu, dout)[0])
+    assert torch.equal(*got)
