@@ -140,7 +140,8 @@ __global__ __launch_bounds__(256) void quant_weights_kernel(const T* __restrict_
 
 // ---- tile scheduler (same contract as the bf16 path) ---------------------------------------------
 __global__ __launch_bounds__(1024) void build_tiles_f8_kernel(const int32_t* __restrict__ gs, int E, int M, int BM,
-                                                              int* __restrict__ count, MTileF8* __restrict__ tiles) {
+                                                              int* __restrict__ count, MTileF8* __restrict__ tiles,
+                                                              FewRows few) {
   __shared__ int wsum[16];
   __shared__ long long wsum64[16];
   __shared__ int s_total[2];
@@ -163,6 +164,12 @@ __global__ __launch_bounds__(1024) void build_tiles_f8_kernel(const int32_t* __r
   const long long start = incl64 - g + wsum64[w];
   const int r0 = (int)min(start, (long long)M), r1 = (int)min(start + g, (long long)M);
   const int nt = (r1 - r0 + BM - 1) / BM;
+  const bool taken = few_rows_take(few, r1 - r0);  // then no tiles are listed
+  if (e == 0) count[3] = taken;
+  if (taken) {
+    if (e == 0) count[0] = 0;
+    return;
+  }
   __syncthreads();
   int incl = nt;
   for (int off = 1; off < 64; off <<= 1) {
@@ -1224,14 +1231,16 @@ static inline int64_t f8_ws_bytes(int64_t M, int64_t E, int64_t BM) {
   return 256 + (ceil_div(M, BM) + E + 1) * (int64_t)sizeof(MTileF8);
 }
 
-// Groups of few rows (decoding): the weight-streaming kernel, with its own row lookup.
-static int launch_fp8_few(const f8::Args& a, const int32_t* gs, int64_t E, bool p2, hipStream_t st) {
+// Groups of few rows (decoding): the weight-streaming kernel, with its own row lookup.  take: where the
+// tile-list kernel writes whether it has the call; nullptr: it has.
+static int launch_fp8_few(const f8::Args& a, const int32_t* gs, int64_t E, bool p2, const int* take, hipStream_t st) {
   Fp8ThinArgs t{};
   t.xq = a.xq;
   t.xs = a.xs;
   t.wq = a.wq;
   t.ws = a.ws;
   t.gs = gs;
+  t.take = take;
   t.out = a.out;
   t.outq = a.outq;
   t.outs = a.outs;
@@ -1246,17 +1255,19 @@ static int launch_fp8_few(const f8::Args& a, const int32_t* gs, int64_t E, bool 
   return launch_fp8_thin(t, p2, st);
 }
 
-// Power-of-two scales (p2): the persistent kernel with the block scales as the MFMA's E8M0
-// operands; it needs K >= 256 and 32-bit operand offsets (MTX_ERR_UNSUPPORTED otherwise).
-template <int EPI>
-static int launch_fp8_v4_p2(const f8::Args& a, const int32_t* gs, int64_t E, int64_t nn, void* ws, hipStream_t st) {
-  const int64_t a_rows = a.gather ? a.gather_rows : a.M;
-  const bool off32 = a_rows * a.K < (int64_t(1) << 32) && (int64_t)a.N * a.K < (int64_t(1) << 32);
-  if (!(off32 && a.K >= 256)) return MTX_ERR_UNSUPPORTED;
-  if (fp8_thin_ok(a.M, E)) return launch_fp8_few(a, gs, E, true, st);
+// The persistent 256-row kernel, or the few-row kernel, or both behind the tile list that chooses.
+template <int EPI, bool P2>
+static int launch_fp8_v4(const f8::Args& a, const int32_t* gs, int64_t E, int64_t nn, void* ws, hipStream_t st) {
+  const FewRowsMode fm = fp8_thin_mode(a.M, E, a.K, a.N, a.I);
+  if (fm == FEW_ALWAYS) return launch_fp8_few(a, gs, E, P2, nullptr, st);
+  const FewRows few = fm == FEW_BY_SIZES ? fp8_thin_rule(a.M, E, a.N, a.I) : FewRows{0, 0, 0};
   int* count = (int*)ws;
   MTileF8* tiles = (MTileF8*)((char*)ws + 256);
-  hipLaunchKernelGGL(f8::build_tiles_f8_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, a.M, 256, count, tiles);
+  hipLaunchKernelGGL(f8::build_tiles_f8_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, a.M, 256, count, tiles, few);
+  if (fm == FEW_BY_SIZES) {
+    const int rc = launch_fp8_few(a, gs, E, P2, count + 3, st);
+    if (rc) return rc;
+  }
   f8::Args b = a;
   b.count = count;
   b.tiles = tiles;
@@ -1264,8 +1275,18 @@ static int launch_fp8_v4_p2(const f8::Args& a, const int32_t* gs, int64_t E, int
   const int ncu = device_cu_count();
   const int64_t cap = ncu > 0 ? round_up(ncu, 8) : 256;
   if (grid > cap) grid = cap;  // persistent: one workgroup per CU (a multiple of the 8 XCDs)
-  hipLaunchKernelGGL((f8::gmm_fp8_v4_kernel<EPI, true>), dim3((unsigned)grid), dim3(512), 0, st, b);
+  hipLaunchKernelGGL((f8::gmm_fp8_v4_kernel<EPI, P2>), dim3((unsigned)grid), dim3(512), 0, st, b);
   return check_launch();
+}
+
+// Power-of-two scales (p2): the persistent kernel with the block scales as the MFMA's E8M0
+// operands; it needs K >= 256 and 32-bit operand offsets (MTX_ERR_UNSUPPORTED otherwise).
+template <int EPI>
+static int launch_fp8_v4_p2(const f8::Args& a, const int32_t* gs, int64_t E, int64_t nn, void* ws, hipStream_t st) {
+  const int64_t a_rows = a.gather ? a.gather_rows : a.M;
+  const bool off32 = a_rows * a.K < (int64_t(1) << 32) && (int64_t)a.N * a.K < (int64_t(1) << 32);
+  if (!(off32 && a.K >= 256)) return MTX_ERR_UNSUPPORTED;
+  return launch_fp8_v4<EPI, true>(a, gs, E, nn, ws, st);
 }
 
 template <int EPI>
@@ -1273,26 +1294,13 @@ static int launch_fp8(const f8::Args& a, const int32_t* gs, int64_t E, int64_t n
   const int64_t a_rows = a.gather ? a.gather_rows : a.M;
   const bool off32 = a_rows * a.K < (int64_t(1) << 32) && (int64_t)a.N * a.K < (int64_t(1) << 32);
   if (a.gather && !(off32 && a.K >= 256)) return MTX_ERR_UNSUPPORTED;  // gathered rows: v4 kernel only
-  if (off32 && a.K >= 256) {
-    if (fp8_thin_ok(a.M, E)) return launch_fp8_few(a, gs, E, false, st);
-    int* count = (int*)ws;
-    MTileF8* tiles = (MTileF8*)((char*)ws + 256);
-    hipLaunchKernelGGL(f8::build_tiles_f8_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, a.M, 256, count, tiles);
-    f8::Args b = a;
-    b.count = count;
-    b.tiles = tiles;
-    int64_t grid = round_up((ceil_div(a.M, 256) + E + 1) * nn, 8);
-    const int ncu = device_cu_count();
-    const int64_t cap = ncu > 0 ? round_up(ncu, 8) : 256;
-    if (grid > cap) grid = cap;  // persistent: one workgroup per CU (a multiple of the 8 XCDs)
-    hipLaunchKernelGGL((f8::gmm_fp8_v4_kernel<EPI>), dim3((unsigned)grid), dim3(512), 0, st, b);
-    return check_launch();
-  }
+  if (off32 && a.K >= 256) return launch_fp8_v4<EPI, false>(a, gs, E, nn, ws, st);
   const bool v3ok = a.K <= 128 * f8::v3::MAX_KB && off32;
   if (v3ok) {
     int* count = (int*)ws;
     MTileF8* tiles = (MTileF8*)((char*)ws + 256);
-    hipLaunchKernelGGL(f8::build_tiles_f8_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, a.M, 256, count, tiles);
+    hipLaunchKernelGGL(f8::build_tiles_f8_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, a.M, 256, count, tiles,
+                       FewRows{0, 0, 0});
     f8::Args b = a;
     b.count = count;
     b.tiles = tiles;
@@ -1303,7 +1311,8 @@ static int launch_fp8(const f8::Args& a, const int32_t* gs, int64_t E, int64_t n
   constexpr int BM = 128, BN = 256;
   int* count = (int*)ws;
   MTileF8* tiles = (MTileF8*)((char*)ws + 256);
-  hipLaunchKernelGGL(f8::build_tiles_f8_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, a.M, BM, count, tiles);
+  hipLaunchKernelGGL(f8::build_tiles_f8_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, a.M, BM, count, tiles,
+                     FewRows{0, 0, 0});
   f8::Args b = a;
   b.count = count;
   b.tiles = tiles;

@@ -43,7 +43,8 @@ struct MTile {
 };
 
 // ---- tile scheduler ---------------------------------------------------------------------------
-// Workspace layout (ints): [0] m-tile count, [1] m-tiles with an expert, [4 .. 11] tickets of the
+// Workspace layout (ints): [0] m-tile count, [1] m-tiles with an expert, [3] whether the few-row kernel
+// takes the call (no m-tiles are listed then), [4 .. 11] tickets of the
 // per-XCD tile queues (zeroed by the tile-list kernel), [16 .. 16+E] group offsets (E+1, clamped to M),
 // [32+E .. ) expert order by descending group size (E), then the MTile array (16B aligned).
 struct GmmWs {
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
                                                            int* __restrict__ count, int* __restrict__ offsets,
                                                            int* __restrict__ order, MTile* __restrict__ tiles,
                                                            int need_order, int* __restrict__ split_cnt, int spread,
-                                                           int align, int merge) {
+                                                           int align, int merge, FewRows few) {
   __shared__ int wsum[16];
   __shared__ long long wsum64[16];
   if (split_cnt && threadIdx.x < kSplitXcd * kSplitMaxRem) split_cnt[threadIdx.x] = 0;
@@ -134,6 +135,12 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
   const int nt = (r1 - r0 + BM - 1) / BM;
   if (e < E) offsets[e] = r0;
   if (e == 0) offsets[E] = min(s_total[0], M);
+  const bool taken = few_rows_take(few, r1 - r0);
+  if (e == 0) count[3] = taken;
+  if (taken) {
+    if (e == 0) count[0] = count[1] = 0;
+    return;
+  }
   __syncthreads();
   // exclusive scan of tile counts
   int incl = nt;
@@ -2481,9 +2488,9 @@ struct MfmaCfg {
 
 static int launch_build_tiles(const int32_t* gs, int64_t E, int64_t M, int BM, const GmmWs& w, hipStream_t st,
                               bool need_order = false, bool reset_split = false, int spread = 0, int align = 0,
-                              int merge = 0) {
+                              int merge = 0, FewRows few = FewRows{0, 0, 0}) {
   hipLaunchKernelGGL(build_tiles_kernel, dim3(1), dim3(1024), 0, st, gs, (int)E, (int)M, BM, w.count, w.offsets,
-                     w.order, w.tiles, need_order ? 1 : 0, reset_split ? w.split_cnt : (int*)nullptr, spread, align, merge);
+                     w.order, w.tiles, need_order ? 1 : 0, reset_split ? w.split_cnt : (int*)nullptr, spread, align, merge, few);
   return check_launch();
 }
 
@@ -2672,9 +2679,9 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
   const bool ring_gather = !gath || (Kred % mf::v3::BKS == 0 && gather_rows * Kred * 2 < (int64_t(1) << 32) &&
                                      Kred * Nout * 2 < (int64_t(1) << 32) &&
                                      ((mode == 2 && I % 128 == 0) || (mode == 0 && Nout % 256 == 0)));
-  if (dtype == MTX_BF16 && aligned && (uintptr_t)out % 16 == 0 && mode != 1 && ring_gather &&
-      gmm_thin_ok(M, E, Kred, Nout, I)) {
-    ThinArgs t;
+  ThinArgs t{};
+  FewRows few{0, 0, 0};
+  if (dtype == MTX_BF16 && aligned && (uintptr_t)out % 16 == 0 && mode != 1 && ring_gather) {
     t.A = (const uint16_t*)x;
     t.W = (const uint16_t*)w;
     t.C = (uint16_t*)out;
@@ -2691,8 +2698,18 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
     // groups of these widths run on
     t.fast_silu = I % 128 == 0 && Kred % mf::BK == 0 && (gath ? gather_rows : M) * Kred * 2 < (int64_t(1) << 32) &&
                   Kred * Nout * 2 < (int64_t(1) << 32);
-    return launch_gmm_thin(t, st);
+    const FewRowsMode fm = gmm_thin_mode(M, E, Kred, Nout, t.I);
+    if (fm == FEW_ALWAYS) return launch_gmm_thin(t, st);
+    if (fm == FEW_BY_SIZES) {
+      few = gmm_thin_rule(M, E, Nout, t.I);
+      t.take = wsp.count + 3;
+    }
   }
+  // the tile list, which also decides between the few-row kernel and the one launched behind both
+  auto build_tiles = [&](int BM, bool reset_split = false, int spread = 0, int align = 0, int merge = 0) -> int {
+    const int rc = launch_build_tiles(gs, E, M, BM, wsp, st, false, reset_split, spread, align, merge, few);
+    return rc != MTX_OK || few.mt == 0 ? rc : launch_gmm_thin(t, st);
+  };
   auto base_args = [&]() {
     mf::Args a;
     a.A = (const uint16_t*)x;
@@ -2747,12 +2764,12 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
         const bool use_w4 = (MTX_W4 & 1) && w4;
         a.vgroup = (use_w4 && merge > 0) ? 1 : 0;
         a.nsplit = ((MTX_NSPLIT & 2) && use_w4 && (I / 128) % 8 == 0) ? 1 : 0;
-        rc = launch_build_tiles(gs, E, M, 256, wsp, st, false, false, spread, align, a.vgroup ? merge : 0);
+        rc = build_tiles(256, false, spread, align, a.vgroup ? merge : 0);
         if (rc) return rc;
         if (use_w4) return launch_w4<mf::FWD, mf::EPI_SWIGLU>(a, gmm_max_tiles(M, E, 256) * (I / 128), st);
         return launch_v3<mf::FWD, mf::EPI_SWIGLU>(a, gmm_max_tiles(M, E, 256) * (I / 128), st);
       }
-      rc = launch_build_tiles(gs, E, M, 128, wsp, st);
+      rc = build_tiles(128);
       if (rc) return rc;
       if (v3ok) return launch_v3_small<mf::FWD, mf::EPI_SWIGLU>(a, gmm_max_tiles(M, E, 128) * (I / 128), st);
       return launch_mfma<128, 256, 1, 2, mf::FWD, mf::EPI_SWIGLU>(a, gmm_max_tiles(M, E, 128) * (I / 128), st);
@@ -2762,7 +2779,7 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
       const int ncu4 = cus_per_xcd();
       if (big_m && !gath && nks >= 4 && short_k && (M / E) >= MTX_V4P_MIN_MEAN && ncu4 >= 1) {
         // short reductions over large groups: persistent workgroups, the ring running across tiles
-        rc = launch_build_tiles(gs, E, M, 256, wsp, st, false, false, spread, align);
+        rc = build_tiles(256, false, spread, align);
         if (rc) return rc;
         const int64_t tiles = gmm_max_tiles(M, E, 256) * (Nout / 256);
         return mode == 0 ? launch_v4p<mf::FWD>(a, tiles, ncu4, st) : launch_v4p<mf::DLHS>(a, tiles, ncu4, st);
@@ -2780,7 +2797,7 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
         }
         const bool use_w4 = ((mode == 0 && (MTX_W4 & 2)) || (mode == 1 && (MTX_W4 & 4))) && w4;
         a.nsplit = ((MTX_NSPLIT & 1) && use_w4 && mode == 0 && (Nout / 256) % 8 == 0) ? 1 : 0;
-        rc = launch_build_tiles(gs, E, M, 256, wsp, st, false, split, spread, align);
+        rc = build_tiles(256, split, spread, align);
         if (rc) return rc;
         // split pieces add at most ncu - rem < ncu workgroups per XCD
         const int64_t grid = round_up(gmm_max_tiles(M, E, 256) * (Nout / 256), 8) + (split ? 8 * (int64_t)ncu : 0);
@@ -2788,7 +2805,7 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
                                      : launch_w4<mf::DLHS, mf::EPI_STORE>(a, grid, st);
         return mode == 0 ? launch_v3<mf::FWD, mf::EPI_STORE>(a, grid, st) : launch_v3<mf::DLHS, mf::EPI_STORE>(a, grid, st);
       }
-      rc = launch_build_tiles(gs, E, M, 128, wsp, st);
+      rc = build_tiles(128);
       if (rc) return rc;
       const int64_t grid = gmm_max_tiles(M, E, 128) * (Nout / 256);
       if (v3ok)
@@ -2807,7 +2824,7 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
     const int64_t edge_tiles = (M / 256 + E) * ceil_div(Nout, 256);
     const bool edge_ahead = M / E >= 256 && edge_tiles >= 512 && Nout >= 640;
     if (mode != 2 && Nout % 128 == 0 && (!v3ok || (uintptr_t)out % 16 != 0 || !edge_ahead)) {
-      rc = launch_build_tiles(gs, E, M, 128, wsp, st);
+      rc = build_tiles(128);
       if (rc) return rc;
       const int64_t grid = gmm_max_tiles(M, E, 128) * (Nout / 128);
       return mode == 0 ? launch_mfma<128, 128, 2, 2, mf::FWD, mf::EPI_STORE>(a, grid, st)
@@ -2832,7 +2849,7 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
       a.split_part = wsp.split_part;
       a.ncu_x = ncu;
     }
-    rc = launch_build_tiles(gs, E, M, 256, wsp, st, false, split, a.gm == 1 ? MTX_SPREAD_MIN : 0);
+    rc = build_tiles(256, split, a.gm == 1 ? MTX_SPREAD_MIN : 0);
     if (rc) return rc;
     const int64_t nn = (mode == 2) ? ceil_div(I, 128) : ceil_div(Nout, 256);
     const int64_t grid = round_up(gmm_max_tiles(M, E, 256) * nn, 8) + (split ? 8 * (int64_t)ncu : 0);
@@ -2841,7 +2858,7 @@ static int gmm_driver(int mode, const void* x, const void* w, const int32_t* gs,
                      : launch_v3_edge<mf::DLHS, mf::EPI_STORE>(a, grid, st);
   }
   // f32, and bf16 widths that are no multiple of 8: the f32 MFMA tiles
-  rc = launch_build_tiles(gs, E, M, kMinBM, wsp, st);
+  rc = build_tiles(kMinBM);
   if (rc) return rc;
   const int64_t ntile_max = gmm_max_tiles(M, E, kMinBM);
   const int64_t gy = (mode == 2) ? ceil_div(I, 32) : ceil_div(Nout, 64);

@@ -39,6 +39,7 @@ __global__ __launch_bounds__(NT) void gmm_fp8_thin_kernel(Fp8ThinArgs p) {
   constexpr int NS = SWIGLU ? 2 : 1;   // weight-scale blocks per chunk
   __shared__ __attribute__((aligned(16))) f32x4 part[CW][NB * TB][64];
   __shared__ float s_amax[MT][CW];
+  if (p.take && *p.take == 0) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kw = wave / CW, cw = wave % CW;
   const int l16 = lane & 15, kq = lane >> 4;
@@ -249,12 +250,28 @@ static int launch(const Fp8ThinArgs& a, int64_t grid, hipStream_t st) {
 // rows the 256-row kernel is ahead, 110 against about 200.
 constexpr int64_t kFp8ThinMaxMean = 12;
 
-bool fp8_thin_ok(int64_t M, int64_t E) {
-  return M >= 1 && M < (1 << 20) && E >= 1 && E <= 1024 && M <= E * kFp8ThinMaxMean;
+static int64_t fp8_thin_mt(int64_t M, int64_t E) { return M <= 2 * E ? 16 : 32; }
+
+// Up to 2^19 outputs (SwiGLU: gate and up columns) it is ahead wherever the rows are, or within 6 % (128
+// groups, 768 x 2048, 256 rows uniform / all on one group: 36 / 51 us and 9 / 17 here / there).  Beyond, the
+// group sizes decide (256 groups, 512 x 4096, 256 rows on one group 27 / 14, uniform 61 / 93), but not with
+// short reductions in a large grid, whose workgroups all end at once if the other kernel has the call
+// (256 groups, 512 x 7168, 256 rows on one 23 / 15).
+FewRowsMode fp8_thin_mode(int64_t M, int64_t E, int64_t K, int64_t N, int64_t I) {
+  if (!(M >= 1 && M < (1 << 20) && E >= 1 && E <= 1024 && M <= E * kFp8ThinMaxMean)) return FEW_NEVER;
+  if (M * N <= 1 << 19) return FEW_ALWAYS;
+  const FewRows r = fp8_thin_rule(M, E, N, I);
+  if ((E < M ? E : M) * r.cols < 192) return FEW_NEVER;
+  return K < 2048 && (int64_t)r.max_tiles * r.cols > 4096 ? FEW_NEVER : FEW_BY_SIZES;
+}
+
+FewRows fp8_thin_rule(int64_t M, int64_t E, int64_t N, int64_t I) {
+  const int64_t mt = fp8_thin_mt(M, E);
+  return {(int)mt, (int)((I > 0 ? I : N) / 128), (int)thin_max_tiles(M, E, mt)};
 }
 
 int launch_fp8_thin(const Fp8ThinArgs& a, bool p2, hipStream_t st) {
-  const int64_t MT = a.M <= 2 * (int64_t)a.E ? 16 : 32;
+  const int64_t MT = fp8_thin_mt(a.M, a.E);
   const int64_t mtiles = thin_max_tiles(a.M, a.E, MT);
   const int64_t grid = mtiles * ((a.I > 0 ? a.I : a.N) / 128);
 #define MTX_F8THIN(S, P) (MT == 16 ? f8thin::launch<S, P, 1>(a, grid, st) : f8thin::launch<S, P, 2>(a, grid, st))

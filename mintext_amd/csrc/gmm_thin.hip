@@ -53,6 +53,7 @@ __global__ __launch_bounds__(NW * 64) void gmm_thin_kernel(ThinArgs p) {
   constexpr bool SWIGLU = FORM != PLAIN;
   constexpr int KW = FORM == WIDE ? NW / 2 : NW;  // waves that share a reduction
   __shared__ __attribute__((aligned(16))) float part[NW][16][PADN];
+  if (p.take && *p.take == 0) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ocols = SWIGLU ? p.I : p.N;
   constexpr int OB = FORM == NARROW ? BN / 2 : BN;  // output columns per workgroup
@@ -205,15 +206,42 @@ static int launch(const ThinArgs& a, int64_t grid, bool stream, hipStream_t st) 
 // 525 / 372.
 constexpr int64_t kThinMaxMean = 16;
 
-bool gmm_thin_ok(int64_t M, int64_t E, int64_t Kred, int64_t N, int64_t I) {
-  if (M < 1 || M >= (1 << 20) || E < 1 || E > 1024) return false;
-  if (Kred < 8 || Kred % 8 || N < 8 || N % 8 || I % 8) return false;
-  return M <= E * kThinMaxMean;
+static int64_t thin_mt(int64_t M, int64_t E) { return M <= 2 * E ? 16 : 32; }
+
+// Without a look at the group sizes it takes the calls in which it is ahead wherever the rows are: up to 16
+// rows (an m-tile for each group), and short reductions while the output is small, where even all rows in
+// one group stream little (2^19 outputs, SwiGLU 2^18 gate and up columns; uniform / all on one group against
+// the ring kernel, us: 256 groups, 4096 x 4096 plain, 128 rows 496 / 568 and 31 / 50, but 512 rows on two groups
+// 66 / 45).  A plain store's reduction past 4096 is split over the chip by the ring kernel, which then leads
+// when few groups have rows (8 groups, 14336 x 4096, 32 rows on one 109 / 79, on all 147 / 228).
+// Elsewhere the group sizes decide, where that costs little beside what it can gain: not on a SwiGLU of
+// less than 128 MB of weights (32 groups, 512 x 1536, 512 rows 24 / 20), nor with short reductions in a large
+// grid, whose workgroups all end at once if the ring kernel has the call (256 groups, 512 x 7168, 256 rows on
+// one 25 / 20), nor on a long plain reduction that fills the chip in the ring kernel too (32 groups,
+// 14336 x 4096, 64 rows 540 / 501).
+FewRowsMode gmm_thin_mode(int64_t M, int64_t E, int64_t Kred, int64_t N, int64_t I) {
+  if (M < 1 || M >= (1 << 20) || E < 1 || E > 1024) return FEW_NEVER;
+  if (Kred < 8 || Kred % 8 || N < 8 || N % 8 || I % 8) return FEW_NEVER;
+  if (M > E * kThinMaxMean) return FEW_NEVER;
+  if (M <= 16 && (I > 0 || Kred <= 8192)) return FEW_ALWAYS;
+  if (Kred <= 4096 && M * N <= (I > 0 ? 1 << 18 : 1 << 19)) return FEW_ALWAYS;
+  const FewRows r = gmm_thin_rule(M, E, N, I);
+  const int64_t groups = E < M ? E : M;
+  if (groups * r.cols < 192) return FEW_NEVER;
+  if (I > 0 && groups * Kred * N * 2 < (int64_t)128 << 20) return FEW_NEVER;
+  if (Kred < 2048 && (int64_t)r.max_tiles * r.cols > 4096) return FEW_NEVER;
+  if (I == 0 && Kred > 8192 && groups * r.cols > 256) return FEW_NEVER;
+  return FEW_BY_SIZES;
+}
+
+FewRows gmm_thin_rule(int64_t M, int64_t E, int64_t N, int64_t I) {
+  const int64_t mt = thin_mt(M, E);
+  return {(int)mt, (int)ceil_div(I > 0 ? I : N, 128), (int)thin_max_tiles(M, E, mt)};
 }
 
 int launch_gmm_thin(const ThinArgs& a, hipStream_t st) {
   // rows per m-tile: 16 when the groups hold a row or two on average, else 32
-  const int64_t MT = a.M <= 2 * (int64_t)a.E ? 16 : 32;
+  const int64_t MT = thin_mt(a.M, a.E);
   const int64_t mtiles = thin_max_tiles(a.M, a.E, MT);
   const int64_t bytes = mtiles * a.Kred * a.N * 2;                   // of weights, at most
   // Half the 256 MB memory-side cache or more: nothing of the weights is found there again by the

@@ -80,6 +80,33 @@ __device__ __forceinline__ ThinRows thin_rows(const int32_t* __restrict__ gs, in
   return t.e == -2 || t.r0 >= t.r1 ? ThinRows{-2, 0, 0} : t;
 }
 
+// A call that the few-row kernel may take: its m-tile rows (0: the call is not offered to it), its
+// 128-column output tiles and the m-tiles its grid has room for.
+struct FewRows {
+  int mt, cols, max_tiles;
+};
+
+// Whether the few-row kernel is to take the call, from the group sizes: it streams the weights of a group
+// once for each of its m-tiles, and needs enough of them to fill the chip.  Asked by the tile-list
+// kernels (all 1024 threads, rows: of the thread's group), which then list no tiles; the few-row kernel,
+// launched behind them, ends at once otherwise.  Where the rows are on a few groups the 256-row kernels
+// are ahead by up to 4.7 times (256 groups of 7168 x 4096, 4096 rows on one of them: 955 / 203 us, on all: 2330
+// / 2437); the choice costs the call one tile list and an empty launch, about 5 us.
+// The lines: 1.25 m-tiles a group (2 m-tiles a group lose up to 2 times, 1 never more than the few-row kernel
+// does by itself), 192 column tiles of 256 CUs (128: 62 / 75 us for 8 groups of 32 rows, 4096 x 4096), and a
+// quarter of the grid's m-tiles in use (8 of 261: its empty workgroups take as long as the call, 24 / 15 us
+// in fp8, 512 x 7168).
+__device__ __forceinline__ bool few_rows_take(const FewRows& f, int rows) {
+  __shared__ int s_tiles;
+  if (f.mt == 0) return false;
+  if (threadIdx.x == 0) s_tiles = 0;
+  const int groups = __syncthreads_count(rows > 0);
+  if (rows > 0) atomicAdd(&s_tiles, (rows + f.mt - 1) / f.mt);
+  __syncthreads();
+  const int t = s_tiles;
+  return 4 * t <= 5 * groups && t * f.cols >= 192 && 4 * t >= f.max_tiles;
+}
+
 // m-tiles of MT rows that M rows in E groups can make: groups with rows, full tiles, the rest.
 inline int64_t thin_max_tiles(int64_t M, int64_t E, int64_t MT) { return (E < M ? E : M) + M / MT + 1; }
 

@@ -85,3 +85,77 @@ def test_bf16_odd_widths(dev, K, N, gs):
     assert rel_err(out[:n], O.gmm(xr, f64(w), gs)[:n]) < TOL and (out[n:] == 0).all()
     assert rel_err(dx[:n], O.gmm(dr, f64(w).transpose(0, 2, 1), gs)[:n]) < TOL and (dx[n:] == 0).all()
     assert rel_err(dw, O.tgmm(xr, dr, gs)) < TOL and (dw[gs == 0] == 0).all()
+
+
+# ---- groups of few rows: which kernel, by the group sizes ----------------------------------------------------
+
+def _concentrated(M, E, k):
+    gs = np.zeros(E, np.int32)
+    gs[E // 2:E // 2 + k] = M // k
+    gs[E // 2] += M - M // k * k
+    return gs
+
+
+# "few": the few-row kernel alone; "spread" / "concentrated": both are launched and the group sizes decide
+# (the kernel that has the call is the one whose tiles are computed: the tile list is empty otherwise)
+FEW = [
+    # M (three rows of no group), E, K, N (SwiGLU: gate and up columns), SwiGLU, launches with rows spread, launches on few groups
+    (16, 8, 4096, 1024, False, "few", "few"),
+    (256, 64, 512, 2048, False, "few", "few"),
+    (512, 64, 512, 2048, False, "both", "both"),
+    (512, 64, 512, 1000, False, "few", "few"),
+    (512, 64, 512, 1032, False, "both", "both"),      # a ring kernel with partial tiles beside it
+    (128, 32, 256, 2048, True, "few", "few"),
+    (256, 32, 256, 2048, True, "ring", "ring"),        # SwiGLU: less than 128 MB of weights
+    (256, 32, 1024, 2048, True, "both", "both"),
+    (130, 32, 1032, 2064, True, "both", "both"),
+    (512, 128, 64, 5120, False, "ring", "ring"),       # a grid of more than 4096 workgroups
+    (12, 4, 8448, 512, False, "ring", "ring"),         # a long plain reduction: too few tiles for the chip
+    (64, 64, 4160, 512, False, "both", "both"),
+]
+
+
+@pytest.mark.parametrize("M,E,K,N,swiglu,spread,concentrated", FEW)
+def test_few_rows_by_group_sizes(dev, M, E, K, N, swiglu, spread, concentrated):
+    from mintext_amd.kernels.grouped_matmul import _gmm_fwd, grouped_matmul_swiglu
+
+    f = grouped_matmul_swiglu if swiglu else _gmm_fwd
+    w = _bf16(dev, E, K, N, std=0.05)
+    w64 = f64(w)
+    for gs, want in ((_uniform(M - 3, E, dev)[0], spread), (_concentrated(M - 3, E, 1), concentrated),
+                     (_concentrated(M - 3, E, 2), concentrated), (np.zeros(E, np.int32), concentrated)):
+        x = _bf16(dev, M, K)
+        n = int(gs.sum())
+        g = torch.from_numpy(gs).to(dev)
+        names = launched(lambda: f(x, w, g))
+        assert ("gmm_thin" in names, "gmm_v3" in names) == (want != "ring", want != "few"), names
+        h = O.gmm(f64(x), w64, gs)
+        i = N // 2
+        ref = h[:, :i] / (1 + np.exp(-h[:, :i])) * h[:, i:] if swiglu else h
+        out = f64(f(x, w, g))
+        assert rel_err(out[:n], ref[:n]) < TOL and (out[n:] == 0).all()
+
+
+@pytest.mark.parametrize("scales", ["amax", "pow2"])
+@pytest.mark.parametrize("M,E,K,N,want", [(256, 64, 256, 2048, "few"), (512, 64, 256, 2048, "both"), (24, 2, 256, 32768, "both")])
+def test_fp8_few_rows_by_group_sizes(dev, scales, M, E, K, N, want):
+    from mintext_amd.kernels.fp8 import (grouped_matmul_fp8, grouped_matmul_fp8_swiglu, quantize_fp8_rows,
+                                         quantize_fp8_weights)
+
+    xq, xs = quantize_fp8_rows(_bf16(dev, M, K), scales=scales)
+    wq, ws = quantize_fp8_weights(_bf16(dev, E, K, N, std=0.05), scales=scales)
+    c = lambda t: t.view(torch.uint8).cpu().numpy() if t.dtype == torch.float8_e4m3fn else t.cpu().numpy()
+    for gs in (_uniform(M - 3, E, dev)[0], _concentrated(M - 3, E, 1), _concentrated(M - 3, E, 2), np.zeros(E, np.int32)):
+        n = int(gs.sum())
+        g = torch.from_numpy(gs).to(dev)
+        f = lambda: grouped_matmul_fp8(xq, xs, wq, ws, g, scales=scales)
+        names = launched(f)
+        assert ("gmm_fp8_thin" in names, "gmm_fp8_v4" in names) == (True, want == "both"), names
+        h = O.gmm_fp8(c(xq), c(xs), c(wq), c(ws), gs)
+        out = f64(f())
+        assert rel_err(out[:n], h[:n]) < TOL and (out[n:] == 0).all()
+        _, ys, yb = grouped_matmul_fp8_swiglu(xq, xs, wq, ws, g, return_bf16=True, scales=scales)
+        i = N // 2
+        b = f64(yb)
+        assert rel_err(b[:n], (h[:, :i] / (1 + np.exp(-h[:, :i])) * h[:, i:])[:n]) < TOL and (b[n:] == 0).all()
+        assert (f64(ys)[n:] == 1).all()
