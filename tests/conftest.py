@@ -53,6 +53,16 @@ def tile_list_workspace_bytes(M: int, E: int) -> int:
     return up(up((48 + 2 * E + 1) * 4, 256) + (-(-M // 64) + E + 1) * 16, 256)
 
 
+def split_pieces(m_tiles: int, n_tiles: int, stages: int, few_stages: int, cus: int = 32) -> int:
+    """Pieces of the split-tail tiles of a launch of 256-row tiles (XCDs with a full share of them): the rule
+    of ``split_pieces`` in gmm.hip, few_stages 16 in the 8-wave kernel and 32 in the one-wave-per-SIMD one."""
+    tiles = -(-m_tiles * n_tiles // 8)
+    rem = tiles % cus
+    if not 0 < rem <= 16 or 2 * rem > cus or stages < 40:
+        return 1
+    return min(4, cus // rem, max(stages // (few_stages if tiles <= 8 else 40), 1))
+
+
 def launched(f) -> str:
     """The names of the kernels that ``f`` launches, one a line."""
     import torch

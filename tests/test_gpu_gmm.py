@@ -323,22 +323,23 @@ def test_tgmm_bf16_sampled_qwen3_shape(dev):
 
 # --------------------------------------------------------------- split tail (256-row tiles)
 SPLIT_SHAPES = [
-    # (group sizes, Kin, Kout): per-XCD tile counts whose last round is sparse, so the tail
-    # tiles run as k-pieces: 8 x 2080 rows, 1 n-tile -> 9 tiles per XCD, each in 3 pieces;
-    # 4 groups of ~9.5k rows (one empty), 2 n-tiles -> 37 tiles per XCD, the last 5 in 4 pieces
-    ([2080] * 8, 1024, 256),
-    ([9472, 0, 9500, 9444 + 9472], 256, 512),
+    # (group sizes, Kred, N): per-XCD tile counts whose last round is sparse, so the tail tiles run
+    # as k-pieces: 8 x 2080 rows, 1 n-tile -> 9 tiles per XCD, each in 2 pieces; 4 groups of ~9.5k rows
+    # (one empty), 2 n-tiles -> 38 tiles per XCD, the last 6 in 2 pieces; one tile per XCD in 4 pieces
+    ([2080] * 8, 2560, 256),
+    ([9472, 0, 9500, 9444 + 9472], 2560, 512),
     ([300, 5, 257, 0, 1], 2048, 256),
 ]
 
 
 @pytest.mark.parametrize("op", ["fwd", "dlhs"])
-@pytest.mark.parametrize("gs,Kin,Kout", SPLIT_SHAPES)
-def test_gmm_split_tail_matches_whole_tiles(dev, gs, Kin, Kout, op):
+@pytest.mark.parametrize("gs,Kred,N", SPLIT_SHAPES)
+def test_gmm_split_tail_matches_whole_tiles(dev, gs, Kred, N, op):
     """The split tail (full workspace) against whole tiles (workspace without the partials
     region) and the float64 oracle: same values to bf16 rounding, deterministic bits."""
     from mintext_amd import _lib as L
 
+    Kin, Kout = (Kred, N) if op == "fwd" else (N, Kred)
     rng = np.random.default_rng(len(gs) + Kin)
     gs = np.asarray(gs, np.int32)
     M, E = int(gs.sum()) + 7, len(gs)  # 7 rows past the groups -> zeros
@@ -366,7 +367,7 @@ def test_gmm_split_tail_matches_whole_tiles(dev, gs, Kin, Kout, op):
 
     split, split2 = run(full), run(full)
     whole = run(full - (64 << 20))  # tile lists only: every tile runs whole
-    assert torch.equal(split, split2)
+    assert torch.equal(split, split2) and not torch.equal(split, whole)  # the tail is split
     xf, wf = xb.float().cpu().numpy(), wb.float().cpu().numpy()
     ref = O.gmm(xf, wf, gs) if op == "fwd" else O.gmm_dlhs(xf, wf, gs)
     assert ref.shape == (M, n_out) and n_red > 0

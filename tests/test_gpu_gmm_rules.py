@@ -159,3 +159,75 @@ def test_fp8_few_rows_by_group_sizes(dev, scales, M, E, K, N, want):
         b = f64(yb)
         assert rel_err(b[:n], (h[:, :i] / (1 + np.exp(-h[:, :i])) * h[:, i:])[:n]) < TOL and (b[n:] == 0).all()
         assert (f64(ys)[n:] == 1).all()
+
+
+# ---- the few-row kernel's wide SwiGLU form (from 512 MB of weights over its m-tiles): 128 gate columns in one half
+# of the waves, the matching up columns in the other; partial columns, a reduction that ends inside a chunk
+@pytest.mark.parametrize("M", [15, 60])
+def test_few_rows_wide_form(dev, M):
+    _wide(dev, M, 16, 1032, 7304, 4)
+
+
+@pytest.mark.parametrize("M,K,I", [(13, 8968, 1032), (32, 4840, 1544)])
+def test_few_rows_wide_form_eight_waves(dev, M, K, I):
+    _wide(dev, M, 16, K, I, 8)
+
+
+def _wide(dev, M, E, K, I, waves):
+    from mintext_amd.kernels.grouped_matmul import grouped_matmul_swiglu
+
+    gs, g = _uniform(M, E, dev)
+    x = _bf16(dev, M + 1, K)
+    x[M] = float("nan")
+    w = torch.empty(E, K, 2 * I, dtype=torch.bfloat16, device=dev).normal_(0.0, 0.02)
+    names = launched(lambda: grouped_matmul_swiglu(x, w, g))
+    tb = 1 if M + 1 <= 2 * E else 2
+    assert f"gmm_thin_kernel<2, {tb}, {waves}," in names, names
+    y = grouped_matmul_swiglu(x, w, g)
+    ref = torch.zeros(M, I, dtype=torch.float64, device=dev)
+    r = 0
+    for e in range(E):
+        h = x[r:r + int(gs[e])].double() @ w[e].double()
+        ref[r:r + int(gs[e])] = torch.nn.functional.silu(h[:, :I]) * h[:, I:]
+        r += int(gs[e])
+    assert rel_err(f64(y[:M]), ref.cpu().numpy()) < TOL and (y[M] == 0).all()
+
+
+# ---- outputs off a 16-byte boundary, which only a caller of the C interface has: 128x128 tiles at any size where
+# the width is a multiple of 128, else single values
+@pytest.mark.parametrize("op", ["fwd", "dlhs", "tgmm"])
+@pytest.mark.parametrize("N", [640, 264])
+def test_outputs_at_any_offset(dev, op, N):
+    from mintext_amd import _lib as L
+
+    E, K, M = 4, 128, 4 * 512
+    if op == "tgmm":
+        E, K, N = 16, N if N % 128 else 1408, 1024
+        M = 40 * E
+    gs, g = _uniform(M, E, dev)
+    x, y = _bf16(dev, M, K), _bf16(dev, M, N)
+    w = _bf16(dev, E, *((K, N) if op == "fwd" else (N, K)), std=0.05)
+    n = E * K * N if op == "tgmm" else M * N
+    ws = L.workspace(L.query("mtx_gmm_workspace_size", M, E), dev)
+    tail = (ws.data_ptr(), ws.numel(), L.stream(dev))
+    outs = []
+    for offset in (0, 1):
+        buf = torch.full((n + offset,), float("nan"), device=dev, dtype=torch.bfloat16)
+        out = buf[offset:]
+        if op == "tgmm":
+            f = lambda: L.call("mtx_tgmm", L.ptr(x), L.ptr(y), L.ptr(g), L.MTX_BF16, M, K, N, E, out.data_ptr(), *tail)
+        else:
+            kin, kout = (K, N) if op == "fwd" else (N, K)
+            code = L.MTX_GMM_OP_FWD if op == "fwd" else L.MTX_GMM_OP_DLHS
+            f = lambda: L.call("mtx_gmm_tiled", code, L.ptr(x), L.ptr(w), L.ptr(g), L.MTX_BF16, M, kin, kout, E, 0, 0,
+                               out.data_ptr(), *tail)
+        names = launched(f)
+        if offset:
+            assert ("gmm_mfma" if N % 128 == 0 and K % 128 == 0 else "f32mm") in names, names
+        outs.append(f64(out))
+    if op == "tgmm":
+        ref = O.tgmm(f64(x), f64(y), gs).ravel()
+    else:
+        ref = O.gmm(f64(x), f64(w) if op == "fwd" else f64(w).transpose(0, 2, 1), gs).ravel()
+    for o in outs:
+        assert rel_err(o, ref) < TOL

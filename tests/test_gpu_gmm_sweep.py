@@ -1,19 +1,20 @@
 """GPU parity sweep of the bf16 grouped GEMM over seeded random shapes (forward and dlhs): expert
 counts 1-48, uniform / Zipf / ragged-with-empty group sizes, rows past sum(group_sizes), and
-reductions on both sides of the persistent kernel's range (Kred <= 1024 runs the persistent
-plain-store kernel, longer ones the per-tile kernel with its split tail).  Each case checks the
-default schedule against the 128-row tiling (the same f32 sums: bit for bit when no tile is split,
-else within a bf16 ulp plus the f32 cancellation error), both against the float64 oracle at
-2e-2, and that rows past the groups are zero.  A second seeded set holds groups of 512 rows or
-more on average with long reductions (forward, dlhs) and the fused SwiGLU: the shapes of the
-one-wave-per-SIMD kernel, with its thin, partial and split-tail tiles."""
+reductions of 128-2048 on the per-tile kernels (with few rows per group the few-row kernel, which
+ignores the tiling).  Each case checks the default schedule against the 128-row tiling (the same
+f32 sums: bit for bit when no tile is split, else within a bf16 ulp plus the f32 cancellation
+error), both against the float64 oracle at 2e-2, and that rows past the groups are zero.  A second
+seeded set holds groups of 512 rows or more on average with long reductions (forward, dlhs) and the
+fused SwiGLU: the shapes of the one-wave-per-SIMD kernel, with its thin, partial and split-tail
+tiles.  A third holds short reductions over groups of 2048 rows or more on average: the persistent
+kernel, with more tiles than workgroups, so that its ring runs across tiles and groups."""
 from __future__ import annotations
 
 import numpy as np
 import pytest
 import torch
 
-from conftest import rel_err
+from conftest import launched, rel_err
 from oracle import moe_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -75,7 +76,7 @@ def test_gmm_sweep(dev, case):
     for o in (out, out128):
         got = o.float().cpu().numpy()
         assert rel_err(got, ref) < 2e-2, rel_err(got, ref)
-    if kred <= 1024:  # persistent kernel: whole tiles, the sums of the 128-row tiling bit for bit
+    if kred <= 1024:  # whole tiles: the sums of the 128-row tiling bit for bit
         assert torch.equal(out, out128)
     else:
         d = (out.float() - out128.float()).abs()
@@ -85,7 +86,7 @@ def test_gmm_sweep(dev, case):
 
 def _cases_large(n=12, seed=4242):
     """Shapes on the one-wave-per-SIMD kernel's side of the dispatch: groups of 512 rows or more
-    on average, reductions past the persistent kernel's 1024 (forward, dlhs) and any reduction
+    on average, reductions past the short ones' 1024 (forward, dlhs) and any reduction
     for the fused SwiGLU (which always takes that kernel at this mean)."""
     rng = np.random.default_rng(seed)
     out = []
@@ -141,6 +142,48 @@ def test_gmm_sweep_large_groups(dev, case):
         d = (out.float() - out128.float()).abs()
         bound = out128.float().abs() * 2.0 ** -7 + 1e-5 * float(np.abs(ref).max())
         assert bool((d <= bound).all()), (d - bound).max().item()
+
+
+def _cases_persistent(n=8, seed=777):
+    """Short reductions (128-1024) over groups of 2048 rows or more on average, more than 256 output tiles:
+    the persistent plain-store kernel."""
+    rng = np.random.default_rng(seed)
+    out = []
+    for i in range(n):
+        E = int(rng.choice([1, 2, 3, 5]))
+        M = E * int(rng.integers(2048, 2700)) + int(rng.integers(0, 256))
+        kred = int(rng.choice([128, 192, 512, 768, 1024]))
+        nout = 256 * -(-(int(rng.choice([300, 520, 700])) * 256) // M)
+        out.append((i, E, M, kred, nout, ("uniform", "zipf", "ragged")[i % 3], int(rng.choice([0, 7, 300])),
+                    "dlhs" if i % 2 else "fwd"))
+    return out
+
+
+@pytest.mark.parametrize("case", _cases_persistent(), ids=lambda c: f"p{c[0]}-E{c[1]}-M{c[2]}-K{c[3]}-N{c[4]}-{c[5]}-p{c[6]}-{c[7]}")
+def test_gmm_sweep_persistent(dev, case):
+    from mintext_amd.kernels.grouped_matmul import _gmm_dlhs, _gmm_fwd
+
+    i, E, M, kred, nout, kind, past, op = case
+    rng = np.random.default_rng(900 + i)
+    gs = _groups(rng, M, E, kind)
+    Mt = M + past
+    xt = torch.from_numpy((rng.standard_normal((Mt, kred)) * 0.5).astype(np.float32)).to(dev).bfloat16()
+    wshape = (E, nout, kred) if op == "dlhs" else (E, kred, nout)
+    wt = torch.from_numpy((rng.standard_normal(wshape) * 0.05).astype(np.float32)).to(dev).bfloat16()
+    gt = torch.from_numpy(gs).to(dev)
+    f = _gmm_dlhs if op == "dlhs" else _gmm_fwd
+    assert "gmm_v4p_kernel" in launched(lambda: f(xt, wt, gt)) and (M // 256) * (nout // 256) > 256
+    out, out128 = f(xt, wt, gt), f(xt, wt, gt, tiling=(128, 1, 256))
+    assert torch.equal(out, out128) and (out[M:] == 0).all()
+    rows = np.sort(rng.choice(M, 512, replace=False))  # sampled rows against float64
+    off = np.concatenate([[0], np.cumsum(gs)])
+    ref = np.empty((512, nout))
+    for r in range(E):
+        at = (rows >= off[r]) & (rows < off[r + 1])
+        w64 = wt[r].double().cpu().numpy()
+        ref[at] = xt[torch.from_numpy(rows[at]).to(dev)].double().cpu().numpy() @ (w64.T if op == "dlhs" else w64)
+    got = out[torch.from_numpy(rows).to(dev)].double().cpu().numpy()
+    assert rel_err(got, ref) < 2.5e-3  # one bf16 rounding
 
 
 def _cases_tgmm(n=6, seed=9090):

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from conftest import rel_err, tile_list_workspace_bytes
+from conftest import rel_err, split_pieces, tile_list_workspace_bytes
 from oracle import moe_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -50,7 +50,7 @@ def test_w4_tile_forms_match_128_row_tiling(dev, op, gi):
     gs = np.asarray(GROUPS[gi], np.int32)
     E = len(gs)
     M = int(gs.sum()) + 300  # two zero tiles past the groups
-    Kred, N = 1280, 512      # 40 ring stages (the per-tile kernels), two 256-column tiles
+    Kred, N = 2560, 512      # 80 ring stages (tails split in two pieces or more), two 256-column tiles
     rng = np.random.default_rng(7 + gi)
     if op == "dlhs":  # dx [M, Kin] = g [M, Kout] @ w[e]^T, w [E, Kin, Kout]
         Kin, Kout = N, Kred
@@ -71,6 +71,9 @@ def test_w4_tile_forms_match_128_row_tiling(dev, op, gi):
     split2 = _run_tiled(dev, op, xb, wb, g, M, Kin, Kout, E, 256, full_ws)
     assert torch.equal(whole, t128), "256-row whole tiles must give the 128-row tiling's bits"
     assert torch.equal(split, split2), "the split tail is deterministic"
+    pieces = 1 if op == "swiglu" else split_pieces(sum(-(-int(n) // 256) for n in gs) + 2, N // 256, Kred // 32, 32)
+    assert op == "swiglu" or gi > 1 or pieces > 1
+    assert pieces == 1 or not torch.equal(split, whole), "the tail is split"
     used = int(gs.sum())
     for out in (whole, split):
         assert (out[used:] == 0).all(), "rows past sum(group_sizes) must be zero"

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from conftest import rel_err, tile_list_workspace_bytes
+from conftest import launched, rel_err, tile_list_workspace_bytes
 from oracle import moe_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -36,11 +36,12 @@ def test_noalloc_gmm_matches_workspace_entry_point(dev, dtype, op):
     lib = L.lib()
     code = {"fwd": L.MTX_GMM_OP_FWD, "swiglu": L.MTX_GMM_OP_SWIGLU, "dlhs": L.MTX_GMM_OP_DLHS}[op]
     stream = L.stream(dev)
-    # bf16 kernel forms, each call smaller than the one before it on that form: reductions of 2304
-    # (beyond the persistent kernel's 32 stages) with >= 512 rows per expert on average (one-wave-
-    # per-SIMD kernel) and then fewer (8-wave per-tile kernel), both with split tails under the full
-    # workspace; then the persistent short-reduction kernel; then 128-row tiles
-    shapes = [(4096, 4, 2304, 2304), (3000, 8, 2304, 2304), (8192, 6, 512, 768), (1000, 3, 256, 384)]
+    # bf16 kernel forms, the second call smaller than the first: reductions of 2560 with >= 512 rows per
+    # expert on average (one-wave-per-SIMD kernel) and then fewer (8-wave per-tile kernel), both with
+    # split tails under the full workspace; then the persistent short-reduction kernel (>= 2048 rows per
+    # expert on average); then 128-row tiles
+    shapes = [(2100, 4, 2560, 2560), (1200, 8, 2560, 2560), (13000, 6, 512, 768), (1000, 3, 256, 384)]
+    kernel = ["gmm_w4", "gmm_v3", "gmm_v4p", "gmm_"]
     for call, (M, E, Kin, Kout) in enumerate(shapes):
         rng = np.random.default_rng(call * 10 + len(op))
         gs = _groups(rng, M, E)
@@ -65,6 +66,11 @@ def test_noalloc_gmm_matches_workspace_entry_point(dev, dtype, op):
             outs[kind] = out
         torch.cuda.synchronize()
         assert torch.equal(outs["noalloc"], outs["tiles"]), f"call {call}: noalloc != tile-list workspace"
+        if dtype == torch.bfloat16 and op != "swiglu":
+            assert kernel[call] in launched(lambda: lib.mtx_gmm_tiled_noalloc(
+                code, x.data_ptr(), w.data_ptr(), g.data_ptr(), L.dtype_code(dtype), M, Kin, Kout, E, 0, 0,
+                outs["noalloc"].data_ptr(), stream))
+            assert torch.equal(outs["tiles"], outs["full"]) == (call > 1), f"call {call}: split tail"
         tol = 2e-2 if dtype == torch.bfloat16 else 1e-5
         f = lambda t: t.double().cpu().numpy()
         assert rel_err(f(outs["noalloc"]), f(outs["full"])) < tol
