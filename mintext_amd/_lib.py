@@ -182,7 +182,7 @@ def plain_forward(*tensors) -> bool:
     """Whether an autograd Function's forward can run without the Function: no gradient is asked for, no
     forward-mode level or functorch transform is active that would have to see (and refuse) it, and no
     jit trace, which records a Function as a call but not the kernels it launches."""
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
         return False
     if torch._C._get_tracing_state() is not None:
         return False

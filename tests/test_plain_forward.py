@@ -14,6 +14,7 @@ def _traced(f, *args):
 def test_plain_forward_conditions():
     x, g = torch.ones(2), torch.ones(2, requires_grad=True)
     assert L.plain_forward(x) and not L.plain_forward(x, g)
+    assert L.plain_forward(x, None) and not L.plain_forward(None, g)  # an operand that is not given
     with torch.no_grad():
         assert L.plain_forward(x, g)
     with torch.autograd.forward_ad.dual_level():
@@ -27,6 +28,16 @@ def test_plain_forward_conditions():
     torch.func.vmap(f)(x)
     _traced(f, x)
     assert seen == [False, False]
+
+
+@pytest.mark.gpu
+def test_unroute_add_without_an_addend(dev):
+    from mintext_amd.kernels import unroute
+    from mintext_amd.kernels.moe_dispatch import unroute_add
+
+    x, w = torch.randn(8, 64, device=dev), torch.rand(4, 2, device=dev)
+    si = torch.arange(8, device=dev, dtype=torch.int32)
+    assert torch.equal(unroute_add(x, si, w, 2, None), unroute(x, si, w, 2))
 
 
 @pytest.mark.gpu
