@@ -187,6 +187,11 @@ __device__ __forceinline__ void store_from_f32(void* p, int64_t i, int dt, float
 }
 
 __device__ __forceinline__ float silu_f32(float g) { return g / (1.0f + expf(-g)); }
+// silu(g) * u with the hardware exp2 / reciprocal (about 1e-6 relative; the GEMM epilogues of whole
+// tiles).  g * u may overflow where the result does not.
+__device__ __forceinline__ float swiglu_fast(float g, float u) {
+  return g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
+}
 
 // Eight consecutive elements p[i .. i+7] as floats and back (i a multiple of 8, p 16-byte
 // aligned): one or two 16-byte accesses, the same conversions as the scalar helpers above.

@@ -981,11 +981,6 @@ __device__ __forceinline__ uint16_t bf16_bits_hw(float f) {
   const __bf16 h = (__bf16)f;  // v_cvt_pk_bf16_f32: round-to-nearest-even
   return __builtin_bit_cast(uint16_t, h);
 }
-// silu(g) * u with the hardware exp2 / reciprocal (about 1e-6 relative; used for bf16 outputs).
-__device__ __forceinline__ float swiglu_fast(float g, float u) {
-  return g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
-}
-
 
 // ---- partial tiles of the split tail ------------------------------------------------------------
 // A piece's f32 tile goes to the workspace and is read by the piece that arrives last, on any XCD.

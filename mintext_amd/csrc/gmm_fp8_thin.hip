@@ -196,8 +196,7 @@ __global__ __launch_bounds__(NT) void gmm_fp8_thin_kernel(Fp8ThinArgs p) {
         for (int j = 0; j < 2; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const float g = acc[j][b][q];
-            y[j][b][q] = g * acc[2 + j][b][q] * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
+            y[j][b][q] = swiglu_fast(acc[j][b][q], acc[2 + j][b][q]);
             m = fmaxf(m, fabsf(y[j][b][q]));
           }
         m = fmaxf(m, __shfl_xor(m, 16));

@@ -26,11 +26,6 @@ constexpr int BN = 128;        // W columns per wave
 constexpr int KC = 32;         // reduction elements per chunk
 constexpr int PADN = BN + 4;   // floats per token row of a wave's partial tile in LDS
 
-// silu(g) * u with the hardware exp2 / reciprocal, as the other bf16 GEMM epilogues
-__device__ __forceinline__ float swiglu_fast(float g, float u) {
-  return g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
-}
-
 // Column J of an 8x8 bf16 block whose row i is in[i]: eight k of one n, an MFMA operand.
 template <int J>
 __device__ __forceinline__ bf16x8 column(const u32x4 (&in)[8]) {
@@ -250,13 +245,13 @@ int launch_gmm_thin(const ThinArgs& a, hipStream_t st) {
   // what does fit (8 rows: 12.6 against 18.1 us).
   const bool stream = bytes >= (int64_t)128 << 20;
   // SwiGLU: 256-byte row pieces of W instead of 128-byte ones (74 rows of 8 groups, 4096 x 2*14336:
-  // 335 -> 306 us), once that leaves enough to do for each wave (64 rows of 128 groups, 2048 x 1536,
-  // 421 MB: 66 against 61 us; 2 rows of 8 groups of 4096 x 28672, 705 MB: 77 against 90)
+  // 335 -> 306 us), once that leaves enough to do for each wave (64 rows of 128 groups, 2048 x 1536, 69
+  // m-tiles, 434 MB: 66 against 59 us; 2 rows of 8 groups of 4096 x 28672, 705 MB: 77 against 90)
   const bool wide = a.I > 0 && bytes >= (int64_t)512 << 20;
   const int64_t nn = wide ? ceil_div(a.I, 128) : a.I > 0 ? ceil_div(a.I, 64) : ceil_div(a.N, 128);
   const int64_t grid = mtiles * nn;
   // few workgroups: eight waves in each instead of four, so that more of the chip's loads are in
-  // flight (64 rows of 128 groups, 768 x 2048, 1072 workgroups: 35 us with eight, 29 with four)
+  // flight (64 rows of 128 groups, 768 x 2048, 1104 workgroups: 35 us with eight, 31 with four)
   const bool eight = grid < 768;
 #define MTX_THIN(F)                                                                                              \
   (MT == 16 ? (eight ? thin::launch<F, 1, 8>(a, grid, stream, st) : thin::launch<F, 1, 4>(a, grid, stream, st))  \
