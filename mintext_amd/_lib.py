@@ -172,10 +172,17 @@ def require_device(*tensors) -> torch.device:
     return dev
 
 
+# Internals of torch that answer without building an object; where one is missing, the public way is taken.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_tracing_state = getattr(torch._C, "_get_tracing_state", None)
+_functorch_level = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", None)
+
+
 def stream(device: torch.device) -> int:
-    """Handle of the current stream of ``device`` (a tensor's, so with an index); asked for on each call,
-    without building a Stream object."""
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    """Handle of the current stream of ``device`` (a tensor's, so with an index); asked for on each call."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def plain_forward(*tensors) -> bool:
@@ -184,9 +191,9 @@ def plain_forward(*tensors) -> bool:
     jit trace, which records a Function as a call but not the kernels it launches."""
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
         return False
-    if torch._C._get_tracing_state() is not None:
+    if _tracing_state is None or _functorch_level is None or _tracing_state() is not None:
         return False
-    return torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+    return getattr(torch.autograd.forward_ad, "_current_level", 0) < 0 and _functorch_level() is None
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:

@@ -30,6 +30,13 @@ def test_plain_forward_conditions():
     assert seen == [False, False]
 
 
+@pytest.mark.parametrize("name", ["_tracing_state", "_functorch_level"])
+def test_without_an_internal_of_torch(monkeypatch, name):
+    """Another torch may not have it: then the Function runs."""
+    monkeypatch.setattr(L, name, None)
+    assert not L.plain_forward(torch.ones(2))
+
+
 @pytest.mark.gpu
 def test_unroute_add_without_an_addend(dev):
     from mintext_amd.kernels import unroute
