@@ -222,8 +222,8 @@ int mtx_tgmm(const void* x, const void* g, const int32_t* group_sizes, int dtype
  * op: MTX_GMM_OP_FWD (out [M,Kout]), MTX_GMM_OP_SWIGLU (Kout = I, w [E,Kin,2I], out [M,I]),
  * MTX_GMM_OP_DLHS (x = g [M,Kout], out = dx [M,Kin]).  tile_m: 0 (shape heuristic), 128 or 256
  * rows per m-tile of the bf16 MFMA path; tile_group: 0 (heuristic) or 1..64 m-tiles per
- * scheduling group.  The f32 path, shapes outside the MFMA tiling and the forward ops with at
- * most 16 rows per group on average (M <= 16 E; one kernel, whatever the tile) ignore both.  Every
+ * scheduling group.  The f32 path, shapes outside the MFMA tiling and the forward calls of at
+ * most 16 rows per group on average (M <= 16 E) that the few-row kernel takes ignore both.  Every
  * configuration computes the same f32 sums; they agree bit for bit unless the split tail
  * (mtx_gmm_workspace_size) splits different tiles, and then to a bf16 rounding.          */
 #define MTX_GMM_OP_FWD    0

@@ -161,6 +161,29 @@ def test_fp8_few_rows_by_group_sizes(dev, scales, M, E, K, N, want):
         assert (f64(ys)[n:] == 1).all()
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+def test_few_rows_choice_under_capture(dev, fp8):
+    """A captured call chooses again in each replay, from the group sizes it finds."""
+    from mintext_amd.kernels.fp8 import grouped_matmul_fp8, quantize_fp8_rows, quantize_fp8_weights
+    from mintext_amd.kernels.grouped_matmul import grouped_matmul
+    from mintext_amd.moe import CapturedLayer
+
+    M, E, K, N = 512, 64, 256, 2048
+    x, w = _bf16(dev, M, K), _bf16(dev, E, K, N, std=0.05)
+    if fp8:
+        (xq, xs), (wq, ws) = quantize_fp8_rows(x), quantize_fp8_weights(w)
+        f = lambda g: grouped_matmul_fp8(xq, xs, wq, ws, g)
+    else:
+        f = lambda g: grouped_matmul(x, w, g)
+    spread, few = _uniform(M - 3, E, dev)[1], torch.from_numpy(_concentrated(M - 3, E, 1)).to(dev)
+    layer = CapturedLayer(f, spread.clone())
+    for g in (spread, few, few, spread, torch.zeros_like(few), few):
+        layer.inputs[0].copy_(g)
+        got = layer.replay().clone()
+        torch.cuda.synchronize()
+        assert torch.equal(got, f(g))
+
+
 # ---- the few-row kernel's wide SwiGLU form (from 512 MB of weights over its m-tiles): 128 gate columns in one half
 # of the waves, the matching up columns in the other; partial columns, a reduction that ends inside a chunk
 @pytest.mark.parametrize("M", [15, 60])
