@@ -252,8 +252,8 @@ constexpr int64_t kFp8ThinMaxMean = 12;
 static int64_t fp8_thin_mt(int64_t M, int64_t E) { return M <= 2 * E ? 16 : 32; }
 
 // Up to 2^19 outputs (SwiGLU: gate and up columns) it is ahead wherever the rows are, or within 6 % (128
-// groups, 768 x 2048, 256 rows uniform / all on one group: 36 / 51 us and 9 / 17 here / there).  Beyond, the
-// group sizes decide (256 groups, 512 x 4096, 256 rows on one group 27 / 14, uniform 61 / 93), but not with
+// groups, 768 x 2048, 256 rows uniform / all on one group: 32 / 56 us and 11 / 17 here / there).  Beyond, the
+// group sizes decide (256 groups, 512 x 4096, 256 rows on one group 27 / 14, uniform 70 / 104), but not with
 // short reductions in a large grid, whose workgroups all end at once if the other kernel has the call
 // (256 groups, 512 x 7168, 256 rows on one 23 / 15).
 FewRowsMode fp8_thin_mode(int64_t M, int64_t E, int64_t K, int64_t N, int64_t I) {

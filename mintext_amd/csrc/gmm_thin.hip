@@ -206,8 +206,8 @@ static int64_t thin_mt(int64_t M, int64_t E) { return M <= 2 * E ? 16 : 32; }
 // Without a look at the group sizes it takes the calls in which it is ahead wherever the rows are: up to 16
 // rows (an m-tile for each group), and short reductions while the output is small, where even all rows in
 // one group stream little (2^19 outputs, SwiGLU 2^18 gate and up columns; uniform / all on one group against
-// the ring kernel, us: 256 groups, 4096 x 4096 plain, 128 rows 496 / 568 and 31 / 50, but 512 rows on two groups
-// 66 / 45).  A plain store's reduction past 4096 is split over the chip by the ring kernel, which then leads
+// the ring kernel, us: 256 groups, 4096 x 4096 plain, 128 rows 520 / 604 and 26 / 47, but 512 rows on two groups
+// 109 / 74).  A plain store's reduction past 4096 is split over the chip by the ring kernel, which then leads
 // when few groups have rows (8 groups, 14336 x 4096, 32 rows on one 109 / 79, on all 147 / 228).
 // Elsewhere the group sizes decide, where that costs little beside what it can gain: not on a SwiGLU of
 // less than 128 MB of weights (32 groups, 512 x 1536, 512 rows 24 / 20), nor with short reductions in a large

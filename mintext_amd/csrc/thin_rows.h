@@ -91,11 +91,11 @@ struct FewRows {
 // kernels (all 1024 threads, rows: of the thread's group), which then list no tiles; the few-row kernel,
 // launched behind them, ends at once otherwise.  Where the rows are on a few groups the 256-row kernels
 // are ahead by up to 4.7 times (256 groups of 7168 x 4096, 4096 rows on one of them: 955 / 203 us, on all: 2330
-// / 2437); the choice costs the call one tile list and an empty launch, about 5 us.
+// / 2437); the choice costs the call one tile list and an empty launch, 5 to 8 us.
 // The lines: 1.25 m-tiles a group (2 m-tiles a group lose up to 2 times, 1 never more than the few-row kernel
-// does by itself), 192 column tiles of 256 CUs (128: 62 / 75 us for 8 groups of 32 rows, 4096 x 4096), and a
-// quarter of the grid's m-tiles in use (8 of 261: its empty workgroups take as long as the call, 24 / 15 us
-// in fp8, 512 x 7168).
+// does by itself), 192 column tiles of 256 CUs (128: 75 us here, 62 there for 256 rows on 8 of 32 groups, SwiGLU of
+// 4096 x 4096), and a quarter of the grid's m-tiles in use (8 of 137: its empty workgroups take as long as the
+// call, 24 us here, 14 there for 128 rows on one of 256 groups, fp8, 512 x 7168).
 __device__ __forceinline__ bool few_rows_take(const FewRows& f, int rows) {
   __shared__ int s_tiles;
   if (f.mt == 0) return false;
